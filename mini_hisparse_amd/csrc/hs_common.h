@@ -163,6 +163,12 @@ __device__ __forceinline__ T wave_inclusive_sum(T v) {
   return v;
 }
 
+// Set bits of a wave's mask below the calling lane.
+__device__ __forceinline__ int32_t lanes_below(uint64_t m) {
+  return static_cast<int32_t>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
+                                                        __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u)));
+}
+
 // Exclusive prefix sum over a 1-D block of up to 1024 threads.  `scratch` must
 // hold 16 elements.  Returns the exclusive prefix; `total` gets the block sum.
 template <typename T>

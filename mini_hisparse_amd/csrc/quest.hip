@@ -374,15 +374,204 @@ __device__ __forceinline__ uint32_t score_key(float s) {
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
-// One workgroup per (query head, request): radix select of the top keys, ties
-// to the lower page, pages written ascending.  When the page keys fit
-// (`KEYS_IN_LDS`), they are computed once into LDS; the digit of each of the
-// four 8-bit passes is found by wave 0 with a suffix scan over the histogram.
-constexpr int64_t QTOPK_LDS_KEYS = 16384;
+// The top keys of one (query head, request) per workgroup, ties to the lower page,
+// pages written ascending; the tail page and the sink are always taken.
+//
+// A thread holds its keys in registers (page j * TT + thread), so the scores are read
+// once.  What bounds the launch is its chain of block-wide steps, so there are few:
+// the least and largest key give a range that one histogram of 2048 equal bins covers
+// (a head's scores crowd into a few powers of two, where fixed top digits of the key put
+// most pages into a handful of bins and a lane's LDS atomics behind each other's), the bin
+// holding the last taken key is found by one scan from the top, and usually holds few
+// keys: they are ranked among themselves.  A bin of more than TOPK_FEW keys is cut into
+// 2048 again; equal keys are ranked by page.  Every wave's taken pages are a ballot, and
+// the ballots of (j, wave) follow the pages' order, so one scan of their counts places
+// each page.
+// Measured (kernel trace, top 64 of 8192 pages, 28 heads x 16 requests): 11.6 us, against
+// 25.8 us for the radix select of four 8-bit digits over keys in LDS; 2048 pages, 14 heads
+// x 4 requests: 5.7 against 10.9 us.
+constexpr int TOPK_BINS = 2048;
+constexpr int TOPK_FEW = 64;
 
-template <bool KEYS_IN_LDS, int TT>
-__global__ __launch_bounds__(TT) void quest_topk_kernel(QuestArgs a) {
-  extern __shared__ uint32_t s_keys[];
+// cnt[0 .. N) -> its exclusive prefix sum, by the first wave.
+template <int N>
+__device__ __forceinline__ void prefix_counts(int32_t* cnt) {
+  constexpr int PER = (N + 63) / 64;
+  const int lane = threadIdx.x;
+  if (threadIdx.x < 64) {
+    int32_t v[PER], own = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      v[i] = lane * PER + i < N ? cnt[lane * PER + i] : 0;
+      own += v[i];
+    }
+    int32_t at = wave_inclusive_sum(own) - own;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      if (lane * PER + i < N) cnt[lane * PER + i] = at;
+      at += v[i];
+    }
+  }
+}
+
+template <int TT, int KPT>
+__global__ __launch_bounds__(TT, 4) void quest_topk_kernel(QuestArgs a) {  // at most 128 VGPRs
+  constexpr int NW = TT / 64, PB = TOPK_BINS / TT;
+  static_assert(KPT * TT <= 32 * TOPK_BINS, "the histogram also holds a bitmap of the pages");
+  __shared__ uint32_t hist[TOPK_BINS];
+  __shared__ uint32_t red[2 * NW];
+  __shared__ uint32_t few_key[TOPK_FEW], few_page[TOPK_FEW];
+  __shared__ int32_t cnt[KPT * NW];
+  __shared__ uint32_t s_bin, s_above, s_held, s_few;
+  const int64_t h = blockIdx.x, b = blockIdx.y;
+  const int32_t T = threadIdx.x, lane = T & 63, wave = T >> 6;
+  int32_t* out = a.pages + b * a.p_sb + h * a.top;
+  if (a.top >= a.count[b]) {
+    for (int64_t j = T; j < a.count[b]; j += TT) out[j] = static_cast<int32_t>(j);
+    return;
+  }
+  const int32_t count = static_cast<int32_t>(a.count[b]);  // at most TT * KPT
+  const float* sc = a.scores + (b * a.Hq + h) * a.cmax;
+  const bool sink = a.keep_sink && a.top > 1;  // top < count: another page than the tail
+  float v[KPT];
+#pragma unroll
+  for (int j = 0; j < KPT; ++j) v[j] = sc[j * TT + T < count ? j * TT + T : 0];
+#pragma unroll
+  for (int i = 0; i < PB; ++i) hist[i * TT + T] = 0u;
+  if (T == 0) s_few = 0u;
+  uint32_t key[KPT];
+  uint32_t live = 0u, taken = 0u;  // bit j: key j may still be taken / is taken
+  uint32_t lo = 0xffffffffu, hi = 0u;
+#pragma unroll
+  for (int j = 0; j < KPT; ++j) {
+    const int32_t p = j * TT + T;
+    key[j] = score_key(v[j]);
+    const bool forced = p == count - 1 || (sink && p == 0);
+    if (forced) taken |= 1u << j;
+    if (p < count && !forced) {
+      live |= 1u << j;
+      lo = key[j] < lo ? key[j] : lo;
+      hi = key[j] > hi ? key[j] : hi;
+    }
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    const uint32_t l = __shfl_xor(lo, off, 64), u = __shfl_xor(hi, off, 64);
+    lo = l < lo ? l : lo;
+    hi = u > hi ? u : hi;
+  }
+  if (lane == 0) {
+    red[wave] = lo;
+    red[NW + wave] = hi;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    lo = red[w] < lo ? red[w] : lo;
+    hi = red[NW + w] > hi ? red[NW + w] : hi;
+  }
+  // still to take among the live keys, all of which lie in [lo, hi]
+  uint32_t need = static_cast<uint32_t>(a.top) - (sink ? 2u : 1u);
+  uint32_t span = hi > lo ? hi - lo : 0u;
+  while (need > 0) {  // the same for the whole workgroup
+    const int bits = 32 - __clz(static_cast<int>(span));  // __clz(0) == 32
+    const int shift = bits > 11 ? bits - 11 : 0;
+#pragma unroll
+    for (int j = 0; j < KPT; ++j)
+      if ((live >> j) & 1u) atomicAdd(&hist[(key[j] - lo) >> shift], 1u);
+    __syncthreads();
+    // thread T owns the PB bins below those of the threads before it
+    uint32_t own[PB], sum = 0u;
+    const int32_t first = TOPK_BINS - 1 - T * PB;
+#pragma unroll
+    for (int i = 0; i < PB; ++i) {
+      own[i] = hist[first - i];
+      sum += own[i];
+    }
+    const uint32_t inc = wave_inclusive_sum(sum);
+    if (lane == 63) red[wave] = inc;
+    __syncthreads();
+    uint32_t above = inc - sum;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) above += w < wave ? red[w] : 0u;
+#pragma unroll
+    for (int i = 0; i < PB; ++i) {
+      if (above < need && above + own[i] >= need) {  // one bin of one thread
+        s_bin = static_cast<uint32_t>(first - i);
+        s_above = above;
+        s_held = own[i];
+      }
+      above += own[i];
+      hist[first - i] = 0u;
+    }
+    __syncthreads();
+    const uint32_t bin = s_bin, held = s_held;
+    need -= s_above;
+#pragma unroll
+    for (int j = 0; j < KPT; ++j) {
+      const uint32_t k = (key[j] - lo) >> shift;
+      if (((live >> j) & 1u) && k >= bin && (k > bin || held == need)) taken |= 1u << j;
+      if (k != bin) live &= ~(1u << j);
+    }
+    if (held == need) break;
+    if (held <= TOPK_FEW) {  // rank the bin's keys among themselves
+#pragma unroll
+      for (int j = 0; j < KPT; ++j)
+        if ((live >> j) & 1u) {
+          const uint32_t i = atomicAdd(&s_few, 1u);
+          few_key[i] = key[j];
+          few_page[i] = static_cast<uint32_t>(j * TT + T);
+        }
+      __syncthreads();
+      if (static_cast<uint32_t>(T) < held) {
+        const uint32_t k = few_key[T], p = few_page[T];
+        uint32_t rank = 0;
+        for (uint32_t i = 0; i < held; ++i) rank += few_key[i] > k || (few_key[i] == k && few_page[i] < p);
+        if (rank < need) atomicOr(&hist[p >> 5], 1u << (p & 31));  // cleared above: a bitmap of the pages
+      }
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < KPT; ++j) taken |= ((hist[(j * TT + T) >> 5] >> (T & 31)) & 1u) << j;
+      break;
+    }
+    if (shift == 0) {  // equal keys: the lowest pages
+      uint64_t m[KPT];
+#pragma unroll
+      for (int j = 0; j < KPT; ++j) {
+        m[j] = __ballot((live >> j) & 1u);
+        if (lane == 0) cnt[j * NW + wave] = __popcll(m[j]);
+      }
+      __syncthreads();
+      prefix_counts<KPT * NW>(cnt);
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < KPT; ++j)
+        if (((live >> j) & 1u) && static_cast<uint32_t>(cnt[j * NW + wave] + lanes_below(m[j])) < need) taken |= 1u << j;
+      __syncthreads();  // cnt is written again below
+      break;
+    }
+    lo += bin << shift;
+    span = (1u << shift) - 1u;
+  }
+  uint64_t m[KPT];
+#pragma unroll
+  for (int j = 0; j < KPT; ++j) {
+    m[j] = __ballot((taken >> j) & 1u);
+    if (lane == 0) cnt[j * NW + wave] = __popcll(m[j]);
+  }
+  __syncthreads();
+  prefix_counts<KPT * NW>(cnt);
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < KPT; ++j)
+    if ((taken >> j) & 1u) out[cnt[j * NW + wave] + lanes_below(m[j])] = j * TT + T;
+}
+
+// The same for histories of more pages than a workgroup's registers hold: a radix
+// select of four 8-bit passes over the scores in memory, each pass's digit found by
+// the first wave with a suffix scan over the histogram.
+__global__ __launch_bounds__(1024) void quest_topk_long_kernel(QuestArgs a) {
+  constexpr int TT = 1024;
   __shared__ uint32_t hist[256];
   __shared__ uint32_t s_prefix, s_mask, s_need;
   __shared__ int64_t scan64[16];
@@ -399,28 +588,6 @@ __global__ __launch_bounds__(TT) void quest_topk_kernel(QuestArgs a) {
     if (p == count - 1 || (sink && p == 0)) return 0xffffffffu;
     return score_key(sc[p]);
   };
-  if constexpr (KEYS_IN_LDS) {
-    // TL scores per thread per round, every load issued before the first key is
-    // stored (a load-then-store loop waits out one load latency per score)
-    constexpr int TL = 8;
-    for (int64_t p0 = threadIdx.x; p0 < count; p0 += static_cast<int64_t>(TT) * TL) {
-      float v[TL];
-#pragma unroll
-      for (int u = 0; u < TL; ++u) {
-        const int64_t p = p0 + static_cast<int64_t>(u) * TT;
-        v[u] = sc[p < count ? p : p0];  // p0 < count: in bounds
-      }
-#pragma unroll
-      for (int u = 0; u < TL; ++u) {
-        const int64_t p = p0 + static_cast<int64_t>(u) * TT;
-        if (p < count) s_keys[p] = (p == count - 1 || (sink && p == 0)) ? 0xffffffffu : score_key(v[u]);
-      }
-    }
-  }
-  auto key_of = [&](int64_t p) -> uint32_t {
-    if constexpr (KEYS_IN_LDS) return s_keys[p];
-    else return key_from_scores(p);
-  };
   if (threadIdx.x == 0) {
     s_prefix = 0u;
     s_mask = 0u;
@@ -433,7 +600,7 @@ __global__ __launch_bounds__(TT) void quest_topk_kernel(QuestArgs a) {
     const uint32_t prefix = s_prefix, mask = s_mask;
     for (int64_t p0 = threadIdx.x - lane; p0 < count; p0 += TT) {  // wave-uniform trip count
       const int64_t p = p0 + lane;
-      const uint32_t k = p < count ? key_of(p) : 0u;
+      const uint32_t k = p < count ? key_from_scores(p) : 0u;
       const uint32_t digit = (k >> shift) & 255u;
       bool pending = p < count && (k & mask) == prefix;
       // Scores of one magnitude share their top digits, so most lanes of a wave
@@ -489,12 +656,12 @@ __global__ __launch_bounds__(TT) void quest_topk_kernel(QuestArgs a) {
   int64_t p1 = p0 + per;
   if (p1 > count) p1 = count;
   int64_t eq = 0;
-  for (int64_t p = p0; p < p1; ++p) eq += key_of(p) == kth;
+  for (int64_t p = p0; p < p1; ++p) eq += key_from_scores(p) == kth;
   int64_t tot;
   const int64_t eq_before = block_exclusive_sum<int64_t>(eq, scan64, &tot);
   int64_t sel = 0, e = eq_before;
   for (int64_t p = p0; p < p1; ++p) {
-    const uint32_t k = key_of(p);
+    const uint32_t k = key_from_scores(p);
     if (k > kth) ++sel;
     else if (k == kth && e++ < static_cast<int64_t>(need_eq)) ++sel;
   }
@@ -502,7 +669,7 @@ __global__ __launch_bounds__(TT) void quest_topk_kernel(QuestArgs a) {
   int64_t o = sel_before;
   e = eq_before;
   for (int64_t p = p0; p < p1; ++p) {
-    const uint32_t k = key_of(p);
+    const uint32_t k = key_from_scores(p);
     bool take = k > kth;
     if (!take && k == kth) take = e++ < static_cast<int64_t>(need_eq);
     if (take) out[o++] = static_cast<int32_t>(p);
@@ -926,23 +1093,23 @@ static int quest_topk_chunk(const void* query, int64_t q_stride_b, int64_t q_str
     }
   }
   const dim3 tgrid(static_cast<unsigned>(heads), static_cast<unsigned>(batch));
-  // 1024 threads per (request, head): measured 22 us against 28 us with 256 at the
-  // microbench shape (4096 pages); HS_TOPK_THREADS=256/512 overrides
-  static const int topk_threads = [] {
-    const char* env = getenv("HS_TOPK_THREADS");
-    const int v = env ? atoi(env) : 0;
-    return v == 256 || v == 512 ? v : 1024;
-  }();
-  const size_t klds = cmax <= QTOPK_LDS_KEYS ? static_cast<size_t>(cmax * 4) : 0;
-  if (cmax <= QTOPK_LDS_KEYS) {
-    if (topk_threads == 256) hipLaunchKernelGGL((quest_topk_kernel<true, 256>), tgrid, dim3(256), klds, stream, a);
-    else if (topk_threads == 512) hipLaunchKernelGGL((quest_topk_kernel<true, 512>), tgrid, dim3(512), klds, stream, a);
-    else hipLaunchKernelGGL((quest_topk_kernel<true, 1024>), tgrid, dim3(1024), klds, stream, a);
-  } else {
-    if (topk_threads == 256) hipLaunchKernelGGL((quest_topk_kernel<false, 256>), tgrid, dim3(256), 0, stream, a);
-    else if (topk_threads == 512) hipLaunchKernelGGL((quest_topk_kernel<false, 512>), tgrid, dim3(512), 0, stream, a);
-    else hipLaunchKernelGGL((quest_topk_kernel<false, 1024>), tgrid, dim3(1024), 0, stream, a);
-  }
+  // The thread count and the keys per thread, by the longest history.  512 threads take up
+  // to 18 keys each in 128 VGPRs, so two workgroups share a CU (8192 pages, 448 heads: 11.6
+  // us, against 13.7 us with 256 threads of 32 keys and 15.5 us with 1024 of 8, which leave
+  // one; 2048 pages, 56 heads: 5.7, 6.3 and 6.2 us).  Longer ones take 1024 threads (8250
+  // pages: 20.6 us, against 23.6 us for 512 threads of 32 keys), and past their registers
+  // the scores are read again for each digit.
+  auto launch = [&](auto kernel, int threads) {
+    hipLaunchKernelGGL(kernel, tgrid, dim3(static_cast<unsigned>(threads)), 0, stream, a);
+  };
+  if (cmax <= 512) launch(quest_topk_kernel<512, 1>, 512);
+  else if (cmax <= 512 * 2) launch(quest_topk_kernel<512, 2>, 512);
+  else if (cmax <= 512 * 4) launch(quest_topk_kernel<512, 4>, 512);
+  else if (cmax <= 512 * 8) launch(quest_topk_kernel<512, 8>, 512);
+  else if (cmax <= 512 * 16) launch(quest_topk_kernel<512, 16>, 512);
+  else if (cmax <= 512 * 18) launch(quest_topk_kernel<512, 18>, 512);
+  else if (cmax <= 1024 * 16) launch(quest_topk_kernel<1024, 16>, 1024);
+  else launch(quest_topk_long_kernel, 1024);
   HS_CHECK_LAUNCH("quest top-k");
   return HS_OK;
 }

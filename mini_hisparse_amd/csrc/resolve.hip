@@ -254,10 +254,6 @@ __device__ __forceinline__ int32_t wave_max_i32(int32_t v) {
   return v;
 }
 
-__device__ __forceinline__ int32_t lanes_below(uint64_t m) {
-  return static_cast<int32_t>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
-                                                        __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u)));
-}
 
 // ---- front: bitmaps, hits and protection, miss ranks, victims, LRU reorder
 // (row_index.py:67-113).  LDS: bits[wl] (selected tokens, then hit tokens),

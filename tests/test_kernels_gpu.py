@@ -423,6 +423,38 @@ def test_quest_topk_with_many_ties_matches_oracle(gpu, pages, top, sink):
     sel = quest_selection(q.to(gpu), lo.to(gpu), hi.to(gpu), length, P, top, keep_sink=sink)
     np.testing.assert_array_equal(sel.device_pages[:, : expected.shape[1]].cpu().numpy(), expected)
 
+def _score_pages(kind, pages, gen):
+    """[pages] page values whose scores crowd, spread or repeat (bf16 exact)."""
+    x = torch.randn(pages, generator=gen)
+    if kind == "spread":  # both signs, 60 decades: the scores' keys span their whole range
+        x = x * 10.0 ** (60 * torch.rand(pages, generator=gen) - 30)
+    elif kind == "crowd":  # one page far above many that lie close together
+        x = 1 + x.abs() / 64
+        x[pages // 2] = 1e30
+    elif kind == "inf":
+        x[:: max(3, pages // 100)] = float("-inf")
+        x[pages // 2] = float("inf")
+    return x.to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("kind", ["normal", "spread", "crowd", "inf"])
+@pytest.mark.parametrize("pages,top", [(2, 1), (66, 65), (512, 8), (513, 8), (1024, 64), (1025, 64), (2048, 3),
+                                       (2049, 64), (4096, 200), (4097, 64), (8192, 64), (8193, 64), (9216, 64),
+                                       (9217, 64), (16384, 5000), (16385, 64)])
+def test_quest_topk_page_counts_and_score_spreads(gpu, kind, pages, top):
+    """Every register variant of the top-k at its first and last page count, over scores that
+    need one cut of their range or several, or fill a bin."""
+    from mini_hisparse_amd.selection import quest_selection
+
+    gen = torch.Generator().manual_seed(pages + top)
+    bounds = torch.zeros(pages, 2, 8, dtype=torch.bfloat16)  # the scores are channel 0's products
+    bounds[:, :, 0] = torch.stack([_score_pages(kind, pages, gen) for _ in range(2)], 1)
+    q = torch.zeros(4, 8, dtype=torch.bfloat16)
+    q[:, 0] = torch.tensor([1.0, 0.5, 1.0, 2.0])
+    expected = oracle.quest_pages(q, bounds, bounds, pages * 16, 16, top)
+    sel = quest_selection(q.to(gpu), bounds.to(gpu), bounds.to(gpu), pages * 16, 16, top)
+    np.testing.assert_array_equal(sel.device_pages[:, : expected.shape[1]].cpu().numpy(), expected)
+
 
 def test_quest_reference_known_answer(gpu):
     """tests/test_selection.py:33-47 of the reference: pages [0, 2], not the mean's page 1."""
