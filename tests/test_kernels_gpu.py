@@ -503,6 +503,20 @@ def test_union_builder_matches_host_adapter(gpu, pages, P, kv, g, top, length):
         np.testing.assert_array_equal(topk.entries.columns[k, : len(cols)].cpu().numpy(), cols)
         np.testing.assert_array_equal(topk.entries.masks[k, : len(cols)].cpu().numpy().astype(np.int64), masks)
 
+@pytest.mark.parametrize(
+    "pages,P,kv,g,top,length",
+    [
+        (400, 16, 1, 1, 256, None),  # union and entries of exactly one chunk (4096)
+        (400, 16, 1, 1, 257, 6385),  # one page more, the last with one token
+        (900, 24, 1, 2, 200, 21590),  # several chunks of pages that are no power of two
+        (6000, 3, 2, 3, 1500, None),  # a head's columns longer than a chunk
+        (260, 16, 1, 16, 16, None),  # many heads of few columns per workgroup
+    ],
+)
+def test_union_builder_chunk_edges(gpu, pages, P, kv, g, top, length):
+    """Unions, entry lists and head columns at the edges of a workgroup's share."""
+    test_union_builder_matches_host_adapter(gpu, pages, P, kv, g, top, length)
+
 
 # --------------------------------------------------------------------- gather
 # rows of 2 KB and 1 KB (one row plane per wave instruction), 256, 128 and 8 bytes (a wave
