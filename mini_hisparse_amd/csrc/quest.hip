@@ -255,24 +255,28 @@ __global__ __launch_bounds__(QT) void quest_score_tile_kernel(QuestArgs a) {
 // zeros, and a sum started at +0 is never -0, so adding either zero leaves it
 // unchanged.  One workgroup scores QP_PAGES pages of one KV head for a chunk of
 // up to QHEADS query heads (wave w: head w, lane l: pages l and l + 64), the
-// bound rows staged in LDS as in quest_score_tile_kernel; two workgroups per
-// CU (4 waves per SIMD).  The KV head is the fastest grid dimension, so the
-// workgroups running together read whole page rows.  Measured at the microbench
-// shape: 37.6 us per launch, against 30.3 us for the loads and LDS stores alone
-// and 26.0 us for the arithmetic alone (LDS reads, VALU and SALU each near
-// their rate: every wave reads the whole tile); tile-fastest or per-XCD grid
-// orders, several tiles per workgroup with the next tile's loads in flight,
-// and a persistent form with two heads per wave and 256-page tiles (2 waves
-// per SIMD) were all slower.  Same arithmetic and order as quest_score_kernel.
+// bound rows staged in LDS as in quest_score_tile_kernel.  The KV head is the fastest grid
+// dimension, so the workgroups running together read whole page rows.
+// The launch is bound by the bounds' HBM stream: what it needs is loads in flight while
+// other waves score.  A 256-byte row (D = 128) is staged in PARTS = 2 halves of 128 bytes,
+// so a workgroup holds 36.9 KB of LDS, four share a CU instead of two, and the second
+// half's loads are in flight while the first is scored.  The bounds are read once per
+// launch, so their loads are non-temporal.  16 requests of 8192 pages, 28 heads, 4 KV heads
+// (268 MB): 66.2 us with whole rows, 55.4 us in halves (page tiles the fastest grid
+// dimension: 54.0), 50.7 us non-temporal = 5.3 TB/s; 8, 4 and 2 requests: 32.0, 19.7 and
+// 13.0 us in halves, 29.4, 18.6 and 12.3 us non-temporal.  Same arithmetic and order as
+// quest_score_kernel.
 constexpr int QP_PAGES = 128;                // pages per workgroup: two per lane
 constexpr int QP_T = 64 * QHEADS;            // one wave per query head of the chunk
 constexpr int QP_UNITS = 4;                  // 16-byte units per thread, bound and staging round
-constexpr int64_t QP_MAX_ROW_BYTES = 256;    // D <= 128: 69.6 KB of LDS, one staging round per tile
+constexpr int64_t QP_MAX_ROW_BYTES = 256;    // D <= 128: one staging round per part
 
-__host__ __device__ constexpr int64_t qp_lds_bytes(int64_t row_bytes) { return 2 * QP_PAGES * (row_bytes + 16); }
+__host__ __device__ constexpr int64_t qp_lds_bytes(int64_t row_bytes, int parts) {
+  return 2 * QP_PAGES * (row_bytes / parts + 16);
+}
 
-template <bool QF32, int DK>
-__global__ __launch_bounds__(QP_T, 4) void quest_score_perm_kernel(QuestArgs a) {  // 4 waves per SIMD: two workgroups per CU
+template <bool QF32, int DK, int PARTS>
+__global__ __launch_bounds__(QP_T, 4 * PARTS) void quest_score_perm_kernel(QuestArgs a) {
 #pragma clang fp contract(off)
   extern __shared__ __attribute__((aligned(16))) unsigned char qp_smem[];
   const int64_t b = blockIdx.z;
@@ -283,7 +287,8 @@ __global__ __launch_bounds__(QP_T, 4) void quest_score_perm_kernel(QuestArgs a) 
   if (a.top >= count || p0 >= count) return;
   const int64_t Hkv = a.Hkv;
   const uint32_t D = DK ? static_cast<uint32_t>(DK) : static_cast<uint32_t>(a.D);
-  const uint32_t rb = D * 2u, rs = rb + 16u, upr = rb / 16u;
+  const uint32_t rb = D * 2u, upr = rb / 16u / PARTS, rs = upr * 16u + 16u;  // units of a row's part, staged row stride
+  constexpr int UNITS = QP_UNITS / PARTS;
   unsigned char* tlo = qp_smem;
   unsigned char* thi = qp_smem + QP_PAGES * rs;
   int64_t npg = count - p0;
@@ -292,37 +297,38 @@ __global__ __launch_bounds__(QP_T, 4) void quest_score_perm_kernel(QuestArgs a) 
   const char* lo_t = static_cast<const char*>(a.kmin[b]) + (p0 * Hkv + kv) * rb;
   const char* hi_t = static_cast<const char*>(a.kmax[b]) + (p0 * Hkv + kv) * rb;
   const uint32_t gstride = static_cast<uint32_t>(Hkv) * rb;  // bytes between consecutive pages
-  {
-    // one staging round (row_bytes <= 256: at most QP_UNITS * QP_T units): every
-    // thread issues its loads before its LDS stores; a unit past the tile reloads
-    // unit 0 (in bounds) and is not stored
-    u32x4 L[QP_UNITS], U[QP_UNITS];
+  // one staging round per part (row_bytes <= 256: at most QP_UNITS * QP_T units in all): a
+  // thread's loads are issued together; a unit past the tile reloads unit 0 (in bounds) and
+  // is not stored
+  u32x4 Ls[UNITS], Us[UNITS];
+  auto load = [&](int part) {
 #pragma unroll
-    for (int k = 0; k < QP_UNITS; ++k) {
+    for (int k = 0; k < UNITS; ++k) {
       uint32_t u = threadIdx.x + static_cast<uint32_t>(k) * QP_T;
       if (u >= units) u = 0;
       const uint32_t r = u / upr, c = u - r * upr;
-      const uint64_t off = static_cast<uint64_t>(r) * gstride + c * 16u;
-      L[k] = *reinterpret_cast<const u32x4*>(lo_t + off);
-      U[k] = *reinterpret_cast<const u32x4*>(hi_t + off);
+      const uint64_t off = static_cast<uint64_t>(r) * gstride + (part * upr + c) * 16u;
+      Ls[k] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(lo_t + off));
+      Us[k] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(hi_t + off));
     }
+  };
+  auto stage = [&]() {
 #pragma unroll
-    for (int k = 0; k < QP_UNITS; ++k) {
+    for (int k = 0; k < UNITS; ++k) {
       const uint32_t u = threadIdx.x + static_cast<uint32_t>(k) * QP_T;
       const uint32_t r = u / upr, c = u - r * upr;
       if (u < units) {
-        *reinterpret_cast<u32x4*>(tlo + r * rs + c * 16u) = L[k];
-        *reinterpret_cast<u32x4*>(thi + r * rs + c * 16u) = U[k];
+        *reinterpret_cast<u32x4*>(tlo + r * rs + c * 16u) = Ls[k];
+        *reinterpret_cast<u32x4*>(thi + r * rs + c * 16u) = Us[k];
       }
     }
-  }
-  __syncthreads();
+  };
+  load(0);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: scalar query loads
   int64_t nh = a.g - hc * QHEADS;
   if (nh > QHEADS) nh = QHEADS;
-  if (wave >= nh) return;  // no barrier follows
-  const int64_t h = kv * a.g + hc * QHEADS + wave;
+  const int64_t h = kv * a.g + hc * QHEADS + (wave < nh ? wave : 0);
   constexpr int QESZ = QF32 ? 4 : 2;
   constexpr int WPU = QF32 ? 8 : 4;  // query words per 16-byte unit of the bounds (8 elements)
   const uint32_t* qw = reinterpret_cast<const uint32_t*>(static_cast<const char*>(a.q) + (b * a.q_sb + h * a.q_sh) * QESZ);
@@ -337,32 +343,42 @@ __global__ __launch_bounds__(QP_T, 4) void quest_score_perm_kernel(QuestArgs a) 
     const bool neg = static_cast<int32_t>(qbits) < 0;
     return half ? (neg ? 0x03020c0cu : 0x07060c0cu) : (neg ? 0x01000c0cu : 0x05040c0cu);
   };
+#pragma unroll
+  for (int part = 0; part < PARTS; ++part) {
+    if (part > 0) __syncthreads();  // every wave has read the part before
+    stage();
+    if (part + 1 < PARTS) load(part + 1);  // in flight while this part is scored
+    __syncthreads();
+    if (wave < nh) {
 #pragma unroll 2
-  for (uint32_t c = 0; c < upr; ++c) {
-    const u32x4 L0 = *reinterpret_cast<const u32x4*>(l0 + c * 16u);
-    const u32x4 L1 = *reinterpret_cast<const u32x4*>(l1 + c * 16u);
-    const u32x4 U0 = *reinterpret_cast<const u32x4*>(u0 + c * 16u);
-    const u32x4 U1 = *reinterpret_cast<const u32x4*>(u1 + c * 16u);
-    uint32_t wq[WPU];
+      for (uint32_t c = 0; c < upr; ++c) {
+        const u32x4 L0 = *reinterpret_cast<const u32x4*>(l0 + c * 16u);
+        const u32x4 L1 = *reinterpret_cast<const u32x4*>(l1 + c * 16u);
+        const u32x4 U0 = *reinterpret_cast<const u32x4*>(u0 + c * 16u);
+        const u32x4 U1 = *reinterpret_cast<const u32x4*>(u1 + c * 16u);
+        uint32_t wq[WPU];
 #pragma unroll
-    for (int i = 0; i < WPU; ++i) wq[i] = qw[c * WPU + i];
+        for (int i = 0; i < WPU; ++i) wq[i] = qw[(part * upr + c) * WPU + i];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const uint32_t qbits = QF32 ? wq[e] : ((e & 1) ? (wq[e >> 1] & 0xffff0000u) : (wq[e >> 1] << 16));
-      const float qf = __uint_as_float(qbits);
-      const uint32_t sel = selector(qbits, e & 1);
-      const float b0 = __uint_as_float(__builtin_amdgcn_perm(U0[e >> 1], L0[e >> 1], sel));
-      const float b1 = __uint_as_float(__builtin_amdgcn_perm(U1[e >> 1], L1[e >> 1], sel));
-      if constexpr (QF32) {
-        const float p0v = qf * b0, p1v = qf * b1;
-        acc0 = acc0 + p0v;
-        acc1 = acc1 + p1v;
-      } else {
-        acc0 = __builtin_fmaf(qf, b0, acc0);
-        acc1 = __builtin_fmaf(qf, b1, acc1);
+        for (int e = 0; e < 8; ++e) {
+          const uint32_t qbits = QF32 ? wq[e] : ((e & 1) ? (wq[e >> 1] & 0xffff0000u) : (wq[e >> 1] << 16));
+          const float qf = __uint_as_float(qbits);
+          const uint32_t sel = selector(qbits, e & 1);
+          const float b0 = __uint_as_float(__builtin_amdgcn_perm(U0[e >> 1], L0[e >> 1], sel));
+          const float b1 = __uint_as_float(__builtin_amdgcn_perm(U1[e >> 1], L1[e >> 1], sel));
+          if constexpr (QF32) {
+            const float p0v = qf * b0, p1v = qf * b1;
+            acc0 = acc0 + p0v;
+            acc1 = acc1 + p1v;
+          } else {
+            acc0 = __builtin_fmaf(qf, b0, acc0);
+            acc1 = __builtin_fmaf(qf, b1, acc1);
+          }
+        }
       }
     }
   }
+  if (wave >= nh) return;
   float* out = a.scores + (b * a.Hq + h) * a.cmax + p0;
   if (lane < npg) out[lane] = acc0;
   if (lane + 64 < npg) out[lane + 64] = acc1;
@@ -1067,17 +1083,17 @@ static int quest_topk_chunk(const void* query, int64_t q_stride_b, int64_t q_str
         query_words && head_dim % 8 == 0 && aligned && row_bytes <= QP_MAX_ROW_BYTES) {
       dim3 grid(static_cast<unsigned>(kv_heads * hchunks), static_cast<unsigned>(ceil_div(cmax, QP_PAGES)),
                 static_cast<unsigned>(batch));
-      const size_t lds = static_cast<size_t>(qp_lds_bytes(row_bytes));
+      const size_t lds = static_cast<size_t>(qp_lds_bytes(row_bytes, head_dim == 128 ? 2 : 1));
       const bool f32q = query_dtype == HS_DTYPE_F32;
       if (head_dim == 128) {
-        if (f32q) hipLaunchKernelGGL((quest_score_perm_kernel<true, 128>), grid, dim3(QP_T), lds, stream, a);
-        else hipLaunchKernelGGL((quest_score_perm_kernel<false, 128>), grid, dim3(QP_T), lds, stream, a);
+        if (f32q) hipLaunchKernelGGL((quest_score_perm_kernel<true, 128, 2>), grid, dim3(QP_T), lds, stream, a);
+        else hipLaunchKernelGGL((quest_score_perm_kernel<false, 128, 2>), grid, dim3(QP_T), lds, stream, a);
       } else if (head_dim == 64) {
-        if (f32q) hipLaunchKernelGGL((quest_score_perm_kernel<true, 64>), grid, dim3(QP_T), lds, stream, a);
-        else hipLaunchKernelGGL((quest_score_perm_kernel<false, 64>), grid, dim3(QP_T), lds, stream, a);
+        if (f32q) hipLaunchKernelGGL((quest_score_perm_kernel<true, 64, 1>), grid, dim3(QP_T), lds, stream, a);
+        else hipLaunchKernelGGL((quest_score_perm_kernel<false, 64, 1>), grid, dim3(QP_T), lds, stream, a);
       } else {
-        if (f32q) hipLaunchKernelGGL((quest_score_perm_kernel<true, 0>), grid, dim3(QP_T), lds, stream, a);
-        else hipLaunchKernelGGL((quest_score_perm_kernel<false, 0>), grid, dim3(QP_T), lds, stream, a);
+        if (f32q) hipLaunchKernelGGL((quest_score_perm_kernel<true, 0, 1>), grid, dim3(QP_T), lds, stream, a);
+        else hipLaunchKernelGGL((quest_score_perm_kernel<false, 0, 1>), grid, dim3(QP_T), lds, stream, a);
       }
       HS_CHECK_LAUNCH("quest scorer");
     } else if (head_dim % epv == 0 && aligned && row_bytes <= QS_MAX_ROW_BYTES) {
