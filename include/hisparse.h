@@ -316,7 +316,7 @@ int hs_rotary_split_append(const void* qkv, int64_t qkv_stride, void* q, void* k
 /*
  * A write of `tokens` consecutive K/V rows to one (request, layer) whose page
  * placement the caller has decided: the page loop of HostStore.append
- * (mini_hisparse/storage.py:273-318) -- prefill or decode -- in one launch per 64
+ * (mini_hisparse/storage.py:273-318) -- prefill or decode -- in one launch per 448
  * pages.
  *   k, v        [tokens, kv_heads, head_dim] in the pool dtype, kv_stride_t elements
  *               between token rows

@@ -306,8 +306,16 @@ extern "C" int hs_rotary_split_append(const void* qkv, int64_t qkv_stride, void*
 
 namespace hs {
 
-constexpr int TMAXP = 64;
+// Pages per launch.  The host mirror's writes bound a long write, and a launch ends only
+// when its last ones have drained over the link, so a long write takes as many pages per
+// launch as the 4 KB of kernel arguments hold: 16384 tokens of 2 KB rows (33.5 MB to the
+// host) took 16 launches of 64 pages, 760 us = 44 GB/s; 3 of 448 take 622 us =
+// 54 GB/s of the pinned copy's 57.  A write of up to 64 pages keeps the small argument
+// block, which every launch copies.
+constexpr int TMAXP = 448;
+constexpr int TFEWP = 64;
 
+template <int PAGES>
 struct TokenAppendArgs {
   const char* k;
   const char* v;
@@ -319,7 +327,7 @@ struct TokenAppendArgs {
   float* summ;  // nullable [pages, Hkv, D] float32
   int64_t P, row_bytes, n_elem, esz;
   int64_t first_page, first_within, tokens;
-  int32_t slot[TMAXP], hslot[TMAXP];
+  int32_t slot[PAGES], hslot[PAGES];
 };
 
 template <int DT>
@@ -337,8 +345,10 @@ __device__ __forceinline__ bool takes_new_max(float old, float x) {
   else return !(old > x);
 }
 
-template <int DT, int U>
-__global__ __launch_bounds__(AT) void append_tokens_kernel(TokenAppendArgs a) {
+static_assert(sizeof(TokenAppendArgs<TMAXP>) <= 4096, "kernel arguments are at most 4 KB");
+
+template <int DT, int U, int PAGES>
+__global__ __launch_bounds__(AT) void append_tokens_kernel(TokenAppendArgs<PAGES> a) {
   typedef typename std::conditional<U == 16, u32x4, unsigned short>::type T;
   const int j = blockIdx.x;
   const int64_t page = a.first_page + j;
@@ -385,6 +395,43 @@ __global__ __launch_bounds__(AT) void append_tokens_kernel(TokenAppendArgs a) {
   }
 }
 
+// The launches of one write, PAGES pages each, in order; every page has been checked.
+template <int PAGES>
+static int append_tokens_launches(TokenAppendArgs<PAGES> a, const int64_t* slots, const int64_t* host_slots,
+                                  int64_t pages, int32_t dtype, bool wide, hipStream_t stream) {
+  const char* const k = a.k;
+  const char* const v = a.v;
+  const int64_t first_page = a.first_page, first_within = a.first_within, tokens = a.tokens;
+  int64_t token = 0;
+  for (int64_t p0 = 0; p0 < pages; p0 += PAGES) {
+    const int64_t n = pages - p0 < PAGES ? pages - p0 : PAGES;
+    const int64_t within = p0 == 0 ? first_within : 0;
+    a.first_page = first_page + p0;
+    a.first_within = within;
+    a.tokens = within + tokens - token < n * a.P ? tokens - token : n * a.P - within;
+    a.k = k + token * a.kv_sb;
+    a.v = v + token * a.kv_sb;
+    for (int64_t i = 0; i < n; ++i) {
+      a.slot[i] = static_cast<int32_t>(slots[p0 + i]);
+      a.hslot[i] = static_cast<int32_t>(host_slots[p0 + i]);
+    }
+    const dim3 grid(static_cast<unsigned>(n));
+    if (dtype == HS_DTYPE_BF16) {
+      if (wide) hipLaunchKernelGGL((append_tokens_kernel<HS_DTYPE_BF16, 16, PAGES>), grid, dim3(AT), 0, stream, a);
+      else hipLaunchKernelGGL((append_tokens_kernel<HS_DTYPE_BF16, 2, PAGES>), grid, dim3(AT), 0, stream, a);
+    } else if (dtype == HS_DTYPE_F16) {
+      if (wide) hipLaunchKernelGGL((append_tokens_kernel<HS_DTYPE_F16, 16, PAGES>), grid, dim3(AT), 0, stream, a);
+      else hipLaunchKernelGGL((append_tokens_kernel<HS_DTYPE_F16, 2, PAGES>), grid, dim3(AT), 0, stream, a);
+    } else {
+      if (wide) hipLaunchKernelGGL((append_tokens_kernel<HS_DTYPE_F32, 16, PAGES>), grid, dim3(AT), 0, stream, a);
+      else hipLaunchKernelGGL((append_tokens_kernel<HS_DTYPE_F32, 2, PAGES>), grid, dim3(AT), 0, stream, a);
+    }
+    HS_CHECK_LAUNCH("append tokens");
+    token += a.tokens;
+  }
+  return HS_OK;
+}
+
 }  // namespace hs
 
 extern "C" int hs_append_tokens(const void* k, const void* v, int64_t kv_stride_t, int64_t tokens, void* pool,
@@ -409,50 +456,28 @@ extern "C" int hs_append_tokens(const void* k, const void* v, int64_t kv_stride_
                  static_cast<long long>(host_slots[p]));
   }
   const int64_t esz = elem_bytes(dtype);
-  TokenAppendArgs a{};
-  a.k = static_cast<const char*>(k);
-  a.v = static_cast<const char*>(v);
-  a.kv_sb = kv_stride_t * esz;
-  a.pool = static_cast<char*>(pool);
-  a.host = static_cast<char*>(const_cast<void*>(host_alias));
-  a.kmin = static_cast<char*>(minimum);
-  a.kmax = static_cast<char*>(maximum);
-  a.summ = summaries;
-  a.P = page_size;
-  a.n_elem = kv_heads * head_dim;
-  a.esz = esz;
-  a.row_bytes = a.n_elem * esz;
+  const int64_t row_bytes = kv_heads * head_dim * esz;
   const uintptr_t align = reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v) |
                           reinterpret_cast<uintptr_t>(pool) | reinterpret_cast<uintptr_t>(host_alias) |
-                          static_cast<uintptr_t>(a.kv_sb) | static_cast<uintptr_t>(a.row_bytes);
+                          static_cast<uintptr_t>(kv_stride_t * esz) | static_cast<uintptr_t>(row_bytes);
   const bool wide = (align & 15) == 0;
-  int64_t token = 0;
-  for (int64_t p0 = 0; p0 < pages; p0 += TMAXP) {
-    const int64_t n = pages - p0 < TMAXP ? pages - p0 : TMAXP;
-    const int64_t within = p0 == 0 ? first_within : 0;
-    a.first_page = first_page + p0;
-    a.first_within = within;
-    const int64_t chunk_tokens = (within + tokens - token) < n * page_size ? tokens - token : n * page_size - within;
-    a.tokens = chunk_tokens;
-    a.k = static_cast<const char*>(k) + token * a.kv_sb;
-    a.v = static_cast<const char*>(v) + token * a.kv_sb;
-    for (int64_t i = 0; i < n; ++i) {
-      a.slot[i] = static_cast<int32_t>(slots[p0 + i]);
-      a.hslot[i] = static_cast<int32_t>(host_slots[p0 + i]);
-    }
-    const dim3 grid(static_cast<unsigned>(n));
-    if (dtype == HS_DTYPE_BF16) {
-      if (wide) hipLaunchKernelGGL((append_tokens_kernel<HS_DTYPE_BF16, 16>), grid, dim3(AT), 0, stream, a);
-      else hipLaunchKernelGGL((append_tokens_kernel<HS_DTYPE_BF16, 2>), grid, dim3(AT), 0, stream, a);
-    } else if (dtype == HS_DTYPE_F16) {
-      if (wide) hipLaunchKernelGGL((append_tokens_kernel<HS_DTYPE_F16, 16>), grid, dim3(AT), 0, stream, a);
-      else hipLaunchKernelGGL((append_tokens_kernel<HS_DTYPE_F16, 2>), grid, dim3(AT), 0, stream, a);
-    } else {
-      if (wide) hipLaunchKernelGGL((append_tokens_kernel<HS_DTYPE_F32, 16>), grid, dim3(AT), 0, stream, a);
-      else hipLaunchKernelGGL((append_tokens_kernel<HS_DTYPE_F32, 2>), grid, dim3(AT), 0, stream, a);
-    }
-    HS_CHECK_LAUNCH("append tokens");
-    token += chunk_tokens;
-  }
-  return HS_OK;
+  auto write = [&](auto a) {
+    a.k = static_cast<const char*>(k);
+    a.v = static_cast<const char*>(v);
+    a.kv_sb = kv_stride_t * esz;
+    a.pool = static_cast<char*>(pool);
+    a.host = static_cast<char*>(const_cast<void*>(host_alias));
+    a.kmin = static_cast<char*>(minimum);
+    a.kmax = static_cast<char*>(maximum);
+    a.summ = summaries;
+    a.P = page_size;
+    a.n_elem = kv_heads * head_dim;
+    a.esz = esz;
+    a.row_bytes = row_bytes;
+    a.first_page = first_page;
+    a.first_within = first_within;
+    a.tokens = tokens;
+    return append_tokens_launches(a, slots, host_slots, pages, dtype, wide, stream);
+  };
+  return pages <= TFEWP ? write(TokenAppendArgs<TFEWP>{}) : write(TokenAppendArgs<TMAXP>{});
 }

@@ -970,3 +970,9 @@ def test_append_tokens_matches_oracle(gpu, dtype, P, kv, D, start, tokens):
     assert torch.equal(host_pinned, expected[1])
     assert torch.equal(lo_d.cpu(), expected[2]) and torch.equal(hi_d.cpu(), expected[3])
     assert torch.equal(summ_d.cpu(), expected[4])
+
+
+@pytest.mark.parametrize("start,pages,spare", [(0, 64, 0), (5, 64, 0), (0, 65, 0), (3, 448, 2), (0, 449, 1), (13, 900, 0)])
+def test_append_tokens_launch_edges(gpu, start, pages, spare):
+    """Writes that fill the short and the long launch exactly, by one page more, and several."""
+    test_append_tokens_matches_oracle(gpu, torch.bfloat16, 16, 1, 8, start, pages * 16 - start - spare)
