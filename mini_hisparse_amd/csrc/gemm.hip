@@ -6,11 +6,11 @@
 // 16 weight rows as the MFMA's M dimension and the (padded) token rows as its
 // N dimension, so the MFMA's output tile is 16 weight rows x 16 tokens.
 //
-// A workgroup (4 waves) owns 16 or 32 weight rows and one K slice; wave w
+// A workgroup (4 or 8 waves) owns 16 or 32 weight rows and one K slice; wave w
 // takes k-steps (of 32) in groups of GU consecutive steps, round-robin over
-// the waves, so within a round the four waves read GU * 4 * 64 contiguous
-// bytes of every row.  Per round a lane issues all of its loads (4 * GU
-// weight fragments, GU token fragments) before the first MFMA.  The waves'
+// the waves, so within a round the waves read GU * 64 contiguous bytes of every
+// row each.  Per round a lane issues all of its loads (GU weight fragments of
+// every row tile, GU token fragments) before the first MFMA.  The waves'
 // partial tiles are summed in LDS.  With one K slice the workgroup adds the
 // bias and writes y; with several (split-K, for tall-K shapes that would
 // otherwise give too few workgroups) it writes partials and
@@ -29,7 +29,7 @@
 
 namespace hs {
 
-constexpr int GM_T = 256;  // threads per workgroup
+constexpr int GM_T = 256;  // threads per workgroup of gemm_finalize_kernel
 
 template <int DT>
 __device__ __forceinline__ f32x4 gemm_mfma(u32x4 a, u32x4 b, f32x4 c) {
@@ -79,7 +79,7 @@ __device__ __forceinline__ float gemm_round(float v) {
   else return f16_bits_to_f32(f32_to_f16_bits(v));
 }
 
-// GM_TILES row tiles of 16 per workgroup, shared by the 4 waves, which split
+// GM_TILES row tiles of 16 per workgroup, shared by its NW waves, which split
 // the slice's k-steps in rounds of GU.  (Measured on MI355X: splitting rows
 // over the waves instead, or double-buffering the rounds in registers, is
 // slower at every decode shape of the Qwen2.5 0.5B/7B/32B projections.)
@@ -94,10 +94,12 @@ __device__ __forceinline__ float gemm_round(float v) {
 // SiLU rounded, then the product (hs_silu_mul).
 // ARGMAX (one K slice): per token the workgroup's best key over its rows, each
 // logit rounded to the dtype after the bias as the plain form stores it.
-template <int DT, int GM_TILES, int GU, bool TILED, bool SWIGLU = false, bool ARGMAX = false>
-__global__ __launch_bounds__(GM_T) void skinny_gemm_kernel(GemmArgs a) {
+template <int DT, int GM_TILES, int NW, bool TILED, bool NT, bool SWIGLU = false, bool ARGMAX = false>
+__global__ __launch_bounds__(64 * NW) void skinny_gemm_kernel(GemmArgs a) {
+  constexpr int GU = 8;  // k-steps of a wave's round
+  constexpr int GM_T = 64 * NW;
   constexpr int GM_ROWS = 16 * GM_TILES;  // weight rows per workgroup
-  __shared__ float red[4][GM_ROWS][17];
+  __shared__ float red[NW][GM_ROWS][17];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c = lane & 15, j = lane >> 4;
   const int64_t n0 = static_cast<int64_t>(blockIdx.x) * GM_ROWS;
@@ -130,7 +132,7 @@ __global__ __launch_bounds__(GM_T) void skinny_gemm_kernel(GemmArgs a) {
   f32x4 acc[GM_TILES];
 #pragma unroll
   for (int t = 0; t < GM_TILES; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int64_t base = s0 + static_cast<int64_t>(wave) * GU; base < s1; base += 4 * GU) {
+  for (int64_t base = s0 + static_cast<int64_t>(wave) * GU; base < s1; base += NW * GU) {
     // every load of the round before the first MFMA; steps past the slice
     // reload its last step (in bounds) and are skipped
     u32x4 wf[GU][GM_TILES], xf[GU];
@@ -141,7 +143,10 @@ __global__ __launch_bounds__(GM_T) void skinny_gemm_kernel(GemmArgs a) {
       const int64_t k = 32 * s;                   // x is row-major
       const int64_t wk = TILED ? 512 * s : k;      // a 16 x 32 block per k-step when tiled
 #pragma unroll
-      for (int t = 0; t < GM_TILES; ++t) wf[u][t] = *reinterpret_cast<const u32x4*>(wrow[t] + wk);
+      for (int t = 0; t < GM_TILES; ++t) {
+        const u32x4* at = reinterpret_cast<const u32x4*>(wrow[t] + wk);
+        wf[u][t] = NT ? __builtin_nontemporal_load(at) : *at;
+      }
       xf[u] = *reinterpret_cast<const u32x4*>(xrow + k);
     }
 #pragma unroll
@@ -158,15 +163,20 @@ __global__ __launch_bounds__(GM_T) void skinny_gemm_kernel(GemmArgs a) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) red[wave][16 * t + 4 * j + i][c] = acc[t][i];
   __syncthreads();
+  auto sum_of = [&](int r, int m) -> float {
+    float v = red[0][r][m];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) v += red[w][r][m];
+    return v;
+  };
   if constexpr (SWIGLU) {
     static_assert(TILED && GM_TILES == 2, "the fused gate/up product takes a gate tile and an up tile");
     for (int idx = threadIdx.x; idx < 16 * 16; idx += GM_T) {
       const int r = idx >> 4, m = idx & 15;
       const int64_t f = static_cast<int64_t>(blockIdx.x) * 16 + r;
       if (m >= a.M || f >= a.F) continue;
-      const float g = gemm_round<DT>((red[0][r][m] + red[1][r][m] + red[2][r][m] + red[3][r][m]) + 0.f);
-      const float u =
-          gemm_round<DT>((red[0][16 + r][m] + red[1][16 + r][m] + red[2][16 + r][m] + red[3][16 + r][m]) + 0.f);
+      const float g = gemm_round<DT>(sum_of(r, m) + 0.f);
+      const float u = gemm_round<DT>(sum_of(16 + r, m) + 0.f);
       const float act = gemm_round<DT>(g / (1.f + expf(-g)));
       store_elem<DT>(a.out, m * a.out_stride + f, act * u);
     }
@@ -180,7 +190,7 @@ __global__ __launch_bounds__(GM_T) void skinny_gemm_kernel(GemmArgs a) {
       unsigned long long key = 0;
       if (n < a.N) {
         const float b = a.bias != nullptr ? load_elem<DT>(a.bias, n) : 0.f;
-        key = argmax_key(gemm_round<DT>((red[0][r][m] + red[1][r][m] + red[2][r][m] + red[3][r][m]) + b), n);
+        key = argmax_key(gemm_round<DT>(sum_of(r, m) + b), n);
       }
       best[r][m] = key;
     }
@@ -203,8 +213,7 @@ __global__ __launch_bounds__(GM_T) void skinny_gemm_kernel(GemmArgs a) {
       const int r = idx >> 4, m = idx & 15;
       const int64_t n = n0 + r;
       if (m >= a.M || n >= a.N) continue;
-      store_partial(a.words + (split * a.M + m) * a.N + n,
-                    red[0][r][m] + red[1][r][m] + red[2][r][m] + red[3][r][m], tag);
+      store_partial(a.words + (split * a.M + m) * a.N + n, sum_of(r, m), tag);
     }
     __shared__ int s_last;
     __syncthreads();
@@ -247,7 +256,7 @@ __global__ __launch_bounds__(GM_T) void skinny_gemm_kernel(GemmArgs a) {
     const int r = idx >> 4, m = idx & 15;
     const int64_t n = n0 + r;
     if (m >= a.M || n >= a.N) continue;
-    const float v = red[0][r][m] + red[1][r][m] + red[2][r][m] + red[3][r][m];
+    const float v = sum_of(r, m);
     if (a.splits > 1) {
       a.part[(split * a.M + m) * a.N + n] = v;
     } else {
@@ -271,14 +280,24 @@ __global__ __launch_bounds__(GM_T) void gemm_finalize_kernel(const float* part, 
 }
 
 // One workgroup per token: the largest of its `blocks` keys, as the vocabulary index.
-__global__ __launch_bounds__(GM_T) void argmax_finalize_kernel(const unsigned long long* keys, int64_t blocks,
-                                                               int64_t* tokens) {
-  __shared__ unsigned long long wave_best[GM_T / 64];
+// Bound by the round trips of its loads: FIN_KEYS keys per thread are loaded together
+// (4752 keys a token: 4.8 us, 9.2 us with 256 threads of one load at a time).
+constexpr int FIN_T = 1024, FIN_KEYS = 8;
+
+__global__ __launch_bounds__(FIN_T) void argmax_finalize_kernel(const unsigned long long* keys, int64_t blocks,
+                                                                int64_t* tokens) {
+  __shared__ unsigned long long wave_best[FIN_T / 64];
   const int64_t m = blockIdx.x;
   unsigned long long key = 0;
-  for (int64_t b = threadIdx.x; b < blocks; b += GM_T) {
-    const unsigned long long v = keys[m * blocks + b];
-    key = v > key ? v : key;
+  for (int64_t b0 = threadIdx.x; b0 < blocks; b0 += FIN_T * FIN_KEYS) {
+    unsigned long long v[FIN_KEYS];
+#pragma unroll
+    for (int i = 0; i < FIN_KEYS; ++i) {
+      const int64_t b = b0 + i * FIN_T;
+      v[i] = keys[m * blocks + (b < blocks ? b : b0)];
+    }
+#pragma unroll
+    for (int i = 0; i < FIN_KEYS; ++i) key = v[i] > key ? v[i] : key;
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
@@ -289,66 +308,96 @@ __global__ __launch_bounds__(GM_T) void argmax_finalize_kernel(const unsigned lo
   __syncthreads();
   if (threadIdx.x == 0) {
 #pragma unroll
-    for (int w = 1; w < GM_T / 64; ++w) key = wave_best[w] > key ? wave_best[w] : key;
+    for (int w = 1; w < FIN_T / 64; ++w) key = wave_best[w] > key ? wave_best[w] : key;
     tokens[m] = static_cast<int64_t>(0xffffffffu - static_cast<uint32_t>(key));
   }
 }
 
 struct GemmPlan {
-  int tiles, gu;
+  int tiles, waves;
+  bool stream;  // non-temporal weight loads
   int64_t blocks, splits, slice_steps;
 };
 
 static int64_t gemm_ceil(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-static int64_t env_or(const char* name, int64_t fallback) {
-  const char* env = getenv(name);
-  return env ? atoll(env) : fallback;
-}
+// Waves of a workgroup: 8 where a wave of 4 would read its k-steps in more than one round
+// (each round is a memory round trip, and a CU with one workgroup has only its own waves'
+// loads in flight), unless there are so many rows that every CU holds several workgroups.
+// 8 rows, us with 4 and with 8 waves: 3584 x 3584 9.8 and 8.5, 896 x 4864 10.5 and 8.3,
+// 3584 x 18944 39.4 and 30.0; 1152 x 896 (7 steps a wave of 4) 3.60 and 3.65.  The same for
+// a projection in one K slice and its fused forms, so their sums agree.
+static int gemm_waves(int64_t N, int64_t slice_steps) { return slice_steps > 32 && N <= 16384 ? 8 : 4; }
 
-// 16-row workgroups up to 1024 of them, else 32-row; rounds of 8 k-steps
-// (the best of 1/2/4 tiles x 2/4/8 steps measured over the Qwen2.5 decode
-// shapes).  Enough K slices for about two workgroups per CU, each slice
-// keeping at least two rounds per wave.  HS_GEMM_TILES / HS_GEMM_GU /
-// HS_GEMM_SPLITS override the choice (read once).
-static GemmPlan plan_gemm(int64_t N, int64_t K) {
-  static const int64_t f_tiles = env_or("HS_GEMM_TILES", 0), f_gu = env_or("HS_GEMM_GU", 0),
-                       f_splits = env_or("HS_GEMM_SPLITS", 0);
-  GemmPlan p{};
-  p.tiles = gemm_ceil(N, 16) <= 1024 ? 1 : 2;
-  if (f_tiles == 1 || f_tiles == 2 || f_tiles == 4) p.tiles = static_cast<int>(f_tiles);
-  p.gu = f_gu == 4 ? 4 : 8;
-  p.blocks = gemm_ceil(N, 16 * p.tiles);
+// Row tiles of 16 per workgroup and K slices.  The weight's stream bounds the launch, a CU
+// reads about 23 bytes per ns, and the launch ends with the CU that reads most: the cost of
+// a plan is the rounds of its workgroups over the 256 CUs times a workgroup's tile-steps
+// (1 KB each), an eighth more with one tile, which reads x twice as often per weight byte.
+// Merging K slices costs about 48 tile-steps (2 us), and pays only within one round or for
+// long slices.  Measured, 8 rows, us before (at least 512 workgroups of 4 waves) and with
+// these plans: 4608 x 3584 12.6 and 12.0, 3584 x 18944 34.2 and 29.6 (two tiles in two slices
+// instead of one in three), 7168 x 5120 21.6 and 15.7, 5120 x 5120 17.2 and 15.6 (two tiles),
+// 5120 x 27648 64.9 and 53.3 (two tiles in three slices), 896 x 4864 9.6 and 7.5 (three
+// slices), 3584 x 3584 9.9 and 8.1.
+static GemmPlan plan_gemm(int64_t N, int64_t K, bool one_slice = false) {
+  constexpr int64_t CUS = 256, X_SHARE = 8, MERGE = 48, LONG_SLICE = 256, MAX_SPLITS = 3;
   const int64_t steps = K / 32;
-  int64_t splits = gemm_ceil(512, p.blocks);
-  const int64_t most = steps / (2 * 4 * p.gu);
-  if (splits > most) splits = most;
-  if (f_splits > 0) splits = f_splits < steps ? f_splits : steps;  // forced: at least one k-step per slice
-  if (splits < 1) splits = 1;
-  p.slice_steps = gemm_ceil(steps, splits);
-  p.splits = gemm_ceil(steps, p.slice_steps);
+  GemmPlan p{};
+  int64_t best = INT64_MAX;
+  for (int64_t s = 1; s <= (one_slice ? 1 : MAX_SPLITS); ++s) {
+    const int64_t slice = gemm_ceil(steps, s), splits = gemm_ceil(steps, slice);
+    if (splits != s) continue;
+    for (int tiles = 2; tiles >= 1; --tiles) {
+      const int64_t blocks = gemm_ceil(N, 16 * tiles);
+      if (splits > 1 && blocks * splits > CUS && slice < LONG_SLICE) continue;
+      const int64_t stream = gemm_ceil(blocks * splits, CUS) * slice * tiles;
+      const int64_t cost = stream + (tiles == 1 ? stream / X_SHARE : 0) + (splits > 1 ? MERGE : 0);
+      if (cost >= best) continue;
+      best = cost;
+      p.tiles = tiles;
+      p.blocks = blocks;
+      p.splits = splits;
+      p.slice_steps = slice;
+    }
+  }
+  p.waves = gemm_waves(N, p.slice_steps);
+  // A weight is read once per step.  Above the 4 MB of an XCD's L2 nothing of it is left
+  // for the next step, and keeping it costs: 2 x 18944 x 3584 52.4 us, non-temporal 48.2;
+  // 3584 x 18944 30.0 and 28.9; 896 x 4864 8.3 and 8.1.  Below, it may still be in a cache:
+  // 1152 x 896 (2 MB) 3.6 us, non-temporal 3.8.
+  p.stream = N * K * 2 > (4 << 20);
   return p;
 }
 
-template <int DT, int TILES, bool TILED, bool ARGMAX>
+template <int DT, int TILES, bool TILED, bool NT, bool ARGMAX>
+static void launch_gemm_waves(const GemmPlan& p, dim3 grid, const GemmArgs& a, hipStream_t s) {
+  if (p.waves == 8) hipLaunchKernelGGL((skinny_gemm_kernel<DT, TILES, 8, TILED, NT, false, ARGMAX>), grid, dim3(512), 0, s, a);
+  else hipLaunchKernelGGL((skinny_gemm_kernel<DT, TILES, 4, TILED, NT, false, ARGMAX>), grid, dim3(256), 0, s, a);
+}
+
+template <int DT, bool TILED, bool NT, bool ARGMAX>
 static void launch_gemm_tiles(const GemmPlan& p, dim3 grid, const GemmArgs& a, hipStream_t s) {
-  if (p.gu == 4) hipLaunchKernelGGL((skinny_gemm_kernel<DT, TILES, 4, TILED, false, ARGMAX>), grid, dim3(GM_T), 0, s, a);
-  else hipLaunchKernelGGL((skinny_gemm_kernel<DT, TILES, 8, TILED, false, ARGMAX>), grid, dim3(GM_T), 0, s, a);
+  if (p.tiles == 1) launch_gemm_waves<DT, 1, TILED, NT, ARGMAX>(p, grid, a, s);
+  else launch_gemm_waves<DT, 2, TILED, NT, ARGMAX>(p, grid, a, s);
 }
 
 template <int DT, bool TILED, bool ARGMAX = false>
 static void launch_gemm(const GemmPlan& p, dim3 grid, const GemmArgs& a, hipStream_t s) {
-  if (p.tiles == 1) launch_gemm_tiles<DT, 1, TILED, ARGMAX>(p, grid, a, s);
-  else if (p.tiles == 2) launch_gemm_tiles<DT, 2, TILED, ARGMAX>(p, grid, a, s);
-  else launch_gemm_tiles<DT, 4, TILED, ARGMAX>(p, grid, a, s);
+  if constexpr (TILED) {  // a row-major weight's loads take half lines: the other half is read later
+    if (p.stream) return launch_gemm_tiles<DT, TILED, true, ARGMAX>(p, grid, a, s);
+  }
+  launch_gemm_tiles<DT, TILED, false, ARGMAX>(p, grid, a, s);
 }
 
-// The argmax form's plan: the plain plan's tiles and rounds, one K slice.
-static GemmPlan plan_argmax(int64_t N, int64_t K) {
-  GemmPlan p = plan_gemm(N, K);
-  p.slice_steps = K / 32;
-  p.splits = 1;
-  return p;
+template <int DT>
+static void launch_swiglu(const GemmPlan& p, dim3 grid, const GemmArgs& a, hipStream_t s) {
+  if (p.waves == 8) {
+    if (p.stream) hipLaunchKernelGGL((skinny_gemm_kernel<DT, 2, 8, true, true, true>), grid, dim3(512), 0, s, a);
+    else hipLaunchKernelGGL((skinny_gemm_kernel<DT, 2, 8, true, false, true>), grid, dim3(512), 0, s, a);
+  } else {
+    if (p.stream) hipLaunchKernelGGL((skinny_gemm_kernel<DT, 2, 4, true, true, true>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((skinny_gemm_kernel<DT, 2, 4, true, false, true>), grid, dim3(256), 0, s, a);
+  }
 }
 
 }  // namespace hs
@@ -463,17 +512,16 @@ extern "C" int hs_skinny_gemm_swiglu_tiled(const void* x, int64_t x_stride, cons
   a.slice_steps = k / 32;
   a.F = ffn;
   const dim3 grid(static_cast<unsigned>(blocks));
-  if (dtype == HS_DTYPE_BF16)
-    hipLaunchKernelGGL((skinny_gemm_kernel<HS_DTYPE_BF16, 2, 8, true, true>), grid, dim3(GM_T), 0, stream, a);
-  else
-    hipLaunchKernelGGL((skinny_gemm_kernel<HS_DTYPE_F16, 2, 8, true, true>), grid, dim3(GM_T), 0, stream, a);
+  const GemmPlan p = plan_gemm(2 * ffn, k, true);  // the plain projection's waves
+  if (dtype == HS_DTYPE_BF16) launch_swiglu<HS_DTYPE_BF16>(p, grid, a, stream);
+  else launch_swiglu<HS_DTYPE_F16>(p, grid, a, stream);
   HS_CHECK_LAUNCH("skinny GEMM swiglu");
   return HS_OK;
 }
 
 extern "C" int64_t hs_skinny_gemm_argmax_workspace_bytes(int64_t rows, int64_t n, int64_t k) {
   if (rows < 1 || n < 1 || k < 32) return 256;
-  return plan_argmax(n, k).blocks * rows * 8 + 256;
+  return plan_gemm(n, k, true).blocks * rows * 8 + 256;
 }
 
 extern "C" int hs_skinny_gemm_argmax_tiled(const void* x, int64_t x_stride, const void* weight_tiles, int64_t n,
@@ -487,7 +535,7 @@ extern "C" int hs_skinny_gemm_argmax_tiled(const void* x, int64_t x_stride, cons
   HS_CHECK_ARG(x && weight_tiles && tokens, "null GEMM pointer");
   HS_CHECK_ARG((reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(weight_tiles) & 15) == 0,
                "x and weight must be 16-byte aligned");
-  const GemmPlan p = plan_argmax(n, k);
+  const GemmPlan p = plan_gemm(n, k, true);
   HS_CHECK_ARG(p.blocks <= 0x7fffffff, "GEMM too large");
   const int64_t need = p.blocks * rows * 8;
   HS_CHECK_ARG(workspace != nullptr && workspace_bytes >= need && (reinterpret_cast<uintptr_t>(workspace) & 7) == 0,
@@ -507,7 +555,7 @@ extern "C" int hs_skinny_gemm_argmax_tiled(const void* x, int64_t x_stride, cons
   if (dtype == HS_DTYPE_BF16) launch_gemm<HS_DTYPE_BF16, true, true>(p, grid, a, stream);
   else launch_gemm<HS_DTYPE_F16, true, true>(p, grid, a, stream);
   HS_CHECK_LAUNCH("skinny GEMM argmax");
-  hipLaunchKernelGGL(argmax_finalize_kernel, dim3(static_cast<unsigned>(rows)), dim3(GM_T), 0, stream, a.keys,
+  hipLaunchKernelGGL(argmax_finalize_kernel, dim3(static_cast<unsigned>(rows)), dim3(FIN_T), 0, stream, a.keys,
                      p.blocks, tokens);
   HS_CHECK_LAUNCH("argmax finalize");
   return HS_OK;

@@ -227,8 +227,7 @@ def linear_swiglu_tiled(x, tiles, ffn, out=None):
     """``silu(x @ gate.T) * (x @ up.T)`` from :func:`tile_gate_up`'s packing, in one launch
     with one K slice.  It has the bits of :func:`linear_tiled` on the packed weight
     followed by :func:`silu_mul` whenever that GEMM also runs in one K slice
-    (``gemm_workspace_bytes(rows, 2 * ffn, K)`` at its minimum of 256, with the default
-    rounds of 8 k-steps); where the GEMM plans split-K (few output rows, long K) the
+    (``gemm_workspace_bytes(rows, 2 * ffn, K)`` at its minimum of 256); where the GEMM plans split-K (few output rows, long K) the
     sums are the same up to fp32 summation order."""
     _swiglu_check(x, tiles, ffn, out)
     y = torch.empty((x.shape[0], ffn), dtype=x.dtype, device=x.device) if out is None else out

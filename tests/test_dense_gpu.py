@@ -327,3 +327,44 @@ def test_in_kernel_split_merge_replays_from_a_captured_graph(gpu):
                      workspace=ws)  # another launch's words and counters in the same bytes
         torch.cuda.synchronize()
         assert torch.equal(got, expected), replay
+
+
+# one round of 4 waves and one k-step more (8 waves), the last row count with 8 waves and the
+# first with 4, one and two row tiles, a weight of 4 MB and a little more, split and whole K
+PLAN_SHAPES = [(512, 1024), (512, 1056), (2048, 1024), (2064, 1024), (4096, 2048), (4112, 2048), (8208, 1056),
+               (16384, 1056), (16416, 1056), (96, 9600)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 9, 16])
+@pytest.mark.parametrize("n,k", PLAN_SHAPES)
+def test_projection_plans_at_their_edges(gpu, rows, n, k):
+    """Every plan of the projection against the fp32 reference, and where it runs in one K
+    slice the fused forms agree with it bit for bit."""
+    from mini_hisparse_amd.dense import (
+        gemm_workspace_bytes, linear_argmax_tiled, linear_swiglu_tiled, linear_tiled, silu_mul, tile_gate_up, tile_weight,
+    )
+
+    test_linear_matches_an_fp32_reference(gpu, torch.bfloat16, rows, n, k, False)
+    if gemm_workspace_bytes(rows, n, k) > 256:
+        return
+    gen = torch.Generator(device=gpu).manual_seed(rows + n + k)
+    x = torch.randn(rows, k, generator=gen, device=gpu).to(torch.bfloat16)
+    w = (torch.randn(n, k, generator=gen, device=gpu) / k**0.5).to(torch.bfloat16)
+    y = linear_tiled(x, tile_weight(w), n)
+    assert torch.equal(linear_argmax_tiled(x, tile_weight(w), n), y.argmax(-1))
+    assert torch.equal(linear_swiglu_tiled(x, tile_gate_up(w, n // 2), n // 2), silu_mul(y))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [16, 32800, 262144, 262176])
+def test_argmax_key_counts(gpu, n):
+    """The argmax's last step at one key per token, several, a full round of its loads and
+    one more; the largest logit planted in the last rows."""
+    from mini_hisparse_amd.dense import linear_argmax_tiled, tile_weight
+
+    w = torch.randn(n, 32, generator=torch.Generator(device=gpu).manual_seed(n), device=gpu).to(torch.bfloat16)
+    x = torch.randn(3, 32, generator=torch.Generator(device=gpu).manual_seed(5), device=gpu).to(torch.bfloat16)
+    for row, at in enumerate((0, n // 2, n - 1)):
+        w[at] = 4 * x[row]
+    assert linear_argmax_tiled(x, tile_weight(w), n).tolist() == [0, n // 2, n - 1]
