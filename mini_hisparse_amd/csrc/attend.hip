@@ -920,7 +920,7 @@ __global__ __launch_bounds__(64 * attend_waves(DP)) void attend_mfma_kernel(Atte
   // is read again.  The barrier orders every wave's stores before the arrival.
   __syncthreads();
   unsigned long long* counter = a.arrivals + (b * Hkv + k) * a.head_chunks + hchunk;
-  if (threadIdx.x == 0) s_last = arrive_last(counter, a.epoch, parts) ? 1 : 0;
+  if (threadIdx.x == 0) s_last = arrive_last(counter, counter0, a.epoch, parts) ? 1 : 0;
   __syncthreads();
   if (!s_last) return;
   const uint32_t tag = group_tag(a.epoch, round);

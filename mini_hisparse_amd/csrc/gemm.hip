@@ -217,7 +217,7 @@ __global__ __launch_bounds__(64 * NW) void skinny_gemm_kernel(GemmArgs a) {
     }
     __shared__ int s_last;
     __syncthreads();
-    if (threadIdx.x == 0) s_last = arrive_last(a.counters + blockIdx.x, a.epoch, a.splits) ? 1 : 0;
+    if (threadIdx.x == 0) s_last = arrive_last(a.counters + blockIdx.x, c0, a.epoch, a.splits) ? 1 : 0;
     __syncthreads();
     if (!s_last) return;
     constexpr int MS = 8;  // slices whose words are loaded together
@@ -340,24 +340,27 @@ static int gemm_waves(int64_t N, int64_t slice_steps) { return slice_steps > 32 
 // 5120 x 27648 64.9 and 53.3 (two tiles in three slices), 896 x 4864 9.6 and 7.5 (three
 // slices), 3584 x 3584 9.9 and 8.1.
 static GemmPlan plan_gemm(int64_t N, int64_t K, bool one_slice = false) {
-  constexpr int64_t CUS = 256, X_SHARE = 8, MERGE = 48, LONG_SLICE = 256, MAX_SPLITS = 3;
-  const int64_t steps = K / 32;
+  // unsigned, with constant divisors: every projection call plans, on the host's time
+  constexpr uint64_t CUS = 256, X_SHARE = 8, MERGE = 48, LONG_SLICE = 256;
+  const uint64_t steps = static_cast<uint64_t>(K) / 32;
+  const uint64_t n[2] = {(static_cast<uint64_t>(N) + 15) / 16, (static_cast<uint64_t>(N) + 31) / 32};
+  const uint64_t slices[3] = {steps, (steps + 1) / 2, (steps + 2) / 3};
   GemmPlan p{};
-  int64_t best = INT64_MAX;
-  for (int64_t s = 1; s <= (one_slice ? 1 : MAX_SPLITS); ++s) {
-    const int64_t slice = gemm_ceil(steps, s), splits = gemm_ceil(steps, slice);
-    if (splits != s) continue;
-    for (int tiles = 2; tiles >= 1; --tiles) {
-      const int64_t blocks = gemm_ceil(N, 16 * tiles);
-      if (splits > 1 && blocks * splits > CUS && slice < LONG_SLICE) continue;
-      const int64_t stream = gemm_ceil(blocks * splits, CUS) * slice * tiles;
-      const int64_t cost = stream + (tiles == 1 ? stream / X_SHARE : 0) + (splits > 1 ? MERGE : 0);
+  uint64_t best = UINT64_MAX;
+  for (uint64_t s = 1; s <= (one_slice ? 1u : 3u); ++s) {
+    const uint64_t slice = slices[s - 1];
+    if (slice * (s - 1) >= steps) break;  // a slice would be empty
+    for (uint64_t tiles = 2; tiles >= 1; --tiles) {
+      const uint64_t blocks = n[tiles - 1];
+      if (s > 1 && blocks * s > CUS && slice < LONG_SLICE) continue;
+      const uint64_t stream = (blocks * s + CUS - 1) / CUS * slice * tiles;
+      const uint64_t cost = stream + (tiles == 1 ? stream / X_SHARE : 0) + (s > 1 ? MERGE : 0);
       if (cost >= best) continue;
       best = cost;
-      p.tiles = tiles;
-      p.blocks = blocks;
-      p.splits = splits;
-      p.slice_steps = slice;
+      p.tiles = static_cast<int>(tiles);
+      p.blocks = static_cast<int64_t>(blocks);
+      p.splits = static_cast<int64_t>(s);
+      p.slice_steps = static_cast<int64_t>(slice);
     }
   }
   p.waves = gemm_waves(N, p.slice_steps);
