@@ -801,7 +801,7 @@ __global__ __launch_bounds__(RT) void resolve_front_kernel(ResolveBatch batch) {
 //   order  (SW WGs / desc)  token words: needs-hot bits, hits among them (a token
 //                           whose slot, written by the match launch, holds its tag:
 //                           slots left by earlier calls hold other tags), misses;
-//                           LRU entries: protected or not, a copy of the LRU;
+//                           LRU entries: a copy of the LRU, each with its protection bit;
 //   place  (SW WGs / desc)  from every workgroup's counts: the miss prefix per word,
 //                           the victims and the new LRU (the same partitions as the
 //                           front's, row_index.py:94-96, 112-113), the totals.
@@ -833,22 +833,25 @@ struct SplitGeom {
 
 __device__ __forceinline__ bool page_bit(const uint32_t* bits, int64_t p) { return (bits[p >> 5] >> (p & 31)) & 1u; }
 
-// sums (and min / max) of one value per thread, published by thread 0
-__device__ __forceinline__ int64_t block_sum64(int64_t v, int64_t* red) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// Each wave's sum of v, in every lane.
+template <typename V>
+__device__ __forceinline__ V wave_sum(V v) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-  __syncthreads();
-  if (lane == 0) red[wave] = v;
-  __syncthreads();
-  int64_t s = 0;
-  for (int u = 0; u < static_cast<int>(blockDim.x >> 6); ++u) s += red[u];
-  return s;
+  return v;
 }
 
+// The launches below are chains of memory round trips, and a barrier of 8 waves costs
+// a good part of one: each launch has one barrier, after every wave has left all of its
+// counts in LDS (match 2, order 6 and place 12 barriers before), and loads that do not
+// depend on each other share a round trip.  us per launch before and now (kernel trace),
+// 16 requests of 131072 tokens and 32768 hot rows: match 7.7 and 7.3, order 10.4 and 8.3,
+// place 7.1 and 6.3; 3 requests of 65536 tokens and 2048 hot rows: 5.2 and 5.0, 8.7 and
+// 7.2, 6.0 and 5.3.
+constexpr int SWAVES = ST / 64;
+
 __global__ __launch_bounds__(ST) void resolve_split_match_kernel(ResolveBatch batch) {
-  __shared__ int64_t red[ST / 64];
-  __shared__ int32_t red_lo[ST / 64], red_hi[ST / 64];
+  __shared__ int32_t red[SWAVES], red_lo[SWAVES], red_hi[SWAVES];
   const hs_resolve_desc& d = batch.d[blockIdx.y];
   const ResolveWs w = ws_of(d);
   const SplitWs x = split_ws_of(d);
@@ -871,7 +874,7 @@ __global__ __launch_bounds__(ST) void resolve_split_match_kernel(ResolveBatch ba
   const int64_t ppad = (g.NPh + 63) / 64 * 64;
   const int64_t pp = ((g.NPh + SW - 1) / SW + 63) / 64 * 64;
   const int64_t p0 = wi * pp, p1 = p0 + pp < ppad ? p0 + pp : ppad;
-  int64_t c_res = 0;
+  int32_t c_res = 0;  // the history's tokens are below 2^21 (the LDS token bitmaps)
   int32_t lo = INT32_MAX, hi = INT32_MIN;
   for (int64_t pb = p0; pb < p1; pb += static_cast<int64_t>(ST) * SPLIT_SLOTS) {
     Regs<int32_t, SPLIT_SLOTS> sv, rv;
@@ -894,7 +897,7 @@ __global__ __launch_bounds__(ST) void resolve_split_match_kernel(ResolveBatch ba
         const int32_t shift = sv[k] - static_cast<int32_t>(p);  // both in [0, 2^31): no overflow
         lo = shift < lo ? shift : lo;
         hi = shift > hi ? shift : hi;
-        if (rv[k] >= 0 && sel) c_res += g.L - p * g.P < g.P ? g.L - p * g.P : g.P;
+        if (rv[k] >= 0 && sel) c_res += static_cast<int32_t>(g.L - p * g.P < g.P ? g.L - p * g.P : g.P);
       }
       const uint64_t m = __ballot(host && sel && rv[k] < 0);
       if ((lane & 31) == 0) x.needpg[p >> 5] = lane ? static_cast<uint32_t>(m >> 32) : static_cast<uint32_t>(m);
@@ -926,13 +929,17 @@ __global__ __launch_bounds__(ST) void resolve_split_match_kernel(ResolveBatch ba
   }
   lo = wave_min_i32(lo);
   hi = wave_max_i32(hi);
+  c_res = wave_sum(c_res);
   if (lane == 0) {
+    red[wave] = c_res;
     red_lo[wave] = lo;
     red_hi[wave] = hi;
   }
-  const int64_t res = block_sum64(c_res, red);  // its barriers order red_lo / red_hi too
+  __syncthreads();
   if (T == 0) {
-    for (int u = 0; u < ST / 64; ++u) {
+    int64_t res = 0;
+    for (int u = 0; u < SWAVES; ++u) {
+      res += red[u];
       lo = red_lo[u] < lo ? red_lo[u] : lo;
       hi = red_hi[u] > hi ? red_hi[u] : hi;
     }
@@ -944,7 +951,7 @@ __global__ __launch_bounds__(ST) void resolve_split_match_kernel(ResolveBatch ba
 
 template <bool L16>
 __global__ __launch_bounds__(ST) void resolve_split_order_kernel(ResolveBatch batch) {
-  __shared__ int64_t red[ST / 64];
+  __shared__ uint64_t red[SWAVES];
   const hs_resolve_desc& d = batch.d[blockIdx.y];
   const ResolveWs w = ws_of(d);
   const SplitWs x = split_ws_of(d);
@@ -966,28 +973,24 @@ __global__ __launch_bounds__(ST) void resolve_split_order_kernel(ResolveBatch ba
   const int64_t wp = (g.wl + SW - 1) / SW, w0 = wi * wp, w1 = w0 + wp < g.wl ? w0 + wp : g.wl;
   const uint32_t ppw = 32u >> g.pshift;  // pages per token word
   const uint32_t pmask = g.P >= 32 ? 0xffffffffu : (1u << g.P) - 1u;
-  int64_t c_hit = 0, c_miss = 0;
-  int64_t c_free = 0;
-  bool lru_done = false;
-  for (int64_t wb = w0; wb < w1 || !lru_done; wb += ST) {
+  // the needs-page bits of token word `wd`, its pages' first at bit 0 (a multiple of ppw: the
+  // word's pages share one bitmap word); word 0's for a word past the history
+  auto needs_of = [&](int64_t wd) -> uint32_t {
+    const int64_t pf = wd < w1 && (wd << 5) < g.L ? (wd << 5) >> g.pshift : 0;
+    return x.needpg[pf >> 5] >> (pf & 31);
+  };
+  const uint32_t np_first = needs_of(w0 + T);  // with the LRU entries' loads
+  // the LRU entries' protection words are used after the token words, so their loads and
+  // the words' slots make one round trip
+  Regs<uint32_t, SPLIT_SLOTS> pw;
+#pragma unroll
+  for (int k = 0; k < SPLIT_SLOTS; ++k) pw[k] = x.prot[(sl[k] < static_cast<uint32_t>(g.S) ? sl[k] : 0u) >> 5];
+  uint32_t c_hit = 0, c_miss = 0, c_free = 0;
+  for (int64_t wb = w0; wb < w1; wb += ST) {
     const int64_t wd = wb + T;
     const int64_t t0 = wd << 5;
     const bool word = wd < w1 && t0 < g.L;
-    // a multiple of ppw: the word's pages share one bitmap word
-    const int64_t pf = word ? t0 >> g.pshift : 0;
-    const uint32_t np = x.needpg[pf >> 5] >> (pf & 31);
-    if (!lru_done) {  // the LRU's protection words, loaded beside the first needs words
-#pragma unroll
-      for (int k = 0; k < SPLIT_SLOTS; ++k) {
-        const int64_t j = e0 + T + static_cast<int64_t>(k) * ST;
-        const uint32_t pw = x.prot[(sl[k] < static_cast<uint32_t>(g.S) ? sl[k] : 0u) >> 5];
-        if (j < e1) {
-          x.lru_snap[j] = static_cast<uint16_t>(sl[k]);
-          c_free += ((pw >> (sl[k] & 31)) & 1u) ? 0 : 1;
-        }
-      }
-      lru_done = true;
-    }
+    const uint32_t np = wb == w0 ? np_first : needs_of(wd);
     if (wd >= w1) continue;
     uint32_t needs = 0u;
     if (word) {
@@ -1024,21 +1027,35 @@ __global__ __launch_bounds__(ST) void resolve_split_order_kernel(ResolveBatch ba
     c_hit += __popc(hitw);
     c_miss += __popc(missw);
   }
-  const int64_t hits = block_sum64(c_hit, red);
-  const int64_t misses = block_sum64(c_miss, red);
-  const int64_t freed = block_sum64(c_free, red);
+#pragma unroll
+  for (int k = 0; k < SPLIT_SLOTS; ++k) {
+    const int64_t j = e0 + T + static_cast<int64_t>(k) * ST;
+    const uint32_t pr = (pw[k] >> (sl[k] & 31)) & 1u;
+    if (j < e1) {
+      x.lru_snap[j] = static_cast<uint16_t>((sl[k] & 0x7fffu) | pr << 15);  // slots are below 32768
+      c_free += 1u - pr;
+    }
+  }
+  // hits, misses and free entries in 21 bits each: a request has fewer than 2^21 tokens
+  // (front_lds_bytes' limit) and at most 32768 hot rows
+  const uint64_t counts = wave_sum(static_cast<uint64_t>(c_hit) | static_cast<uint64_t>(c_miss) << 21 |
+                                   static_cast<uint64_t>(c_free) << 42);
+  if ((T & 63) == 0) red[T >> 6] = counts;
+  __syncthreads();
   if (T == 0) {
-    x.part[PART_HIT * SPLIT_MAX + wi] = hits;
-    x.part[PART_MISS * SPLIT_MAX + wi] = misses;
-    x.part[PART_FREE * SPLIT_MAX + wi] = freed;
+    uint64_t sum = 0;
+    for (int u = 0; u < SWAVES; ++u) sum += red[u];
+    x.part[PART_HIT * SPLIT_MAX + wi] = static_cast<int64_t>(sum & 0x1fffffu);
+    x.part[PART_MISS * SPLIT_MAX + wi] = static_cast<int64_t>(sum >> 21 & 0x1fffffu);
+    x.part[PART_FREE * SPLIT_MAX + wi] = static_cast<int64_t>(sum >> 42);
   }
 }
 
 template <bool L16>
 __global__ __launch_bounds__(ST) void resolve_split_place_kernel(ResolveBatch batch) {
   __shared__ int64_t s_tot[8];  // resident, hits, misses, unprotected; miss and unprotected offsets; lo; hi
-  __shared__ int32_t scan32[ST / 64];
-  __shared__ int32_t wcnt[ST / 64];
+  __shared__ int32_t wmiss[SWAVES];               // misses in the words of each wave's runs
+  __shared__ int32_t wfree[SPLIT_SLOTS * SWAVES];  // unprotected entries of (row, wave)
   const hs_resolve_desc& d = batch.d[blockIdx.y];
   const ResolveWs w = ws_of(d);
   const SplitWs x = split_ws_of(d);
@@ -1087,6 +1104,22 @@ __global__ __launch_bounds__(ST) void resolve_split_place_kernel(ResolveBatch ba
       s_tot[7] = hi;
     }
   }
+  // the misses of the thread's run of words, and the unprotected LRU entries per (row, wave)
+  const int32_t S = g.S;
+  int32_t cnt = a0 < a1 ? __popc(first_miss) : 0;
+  for (int64_t wd = a0 + 1; wd < a1; ++wd) cnt += __popc(w.missbits[wd]);
+  const int32_t cnt_inc = wave_inclusive_sum(cnt);
+  if (lane == 63) wmiss[wave] = cnt_inc;
+  Regs<bool, SPLIT_SLOTS> fr;
+  Regs<uint64_t, SPLIT_SLOTS> frm;
+#pragma unroll
+  for (int k = 0; k < SPLIT_SLOTS; ++k) {
+    const int64_t j = e0 + T + static_cast<int64_t>(k) * ST;
+    fr[k] = j < e1 && !(sl[k] >> 15);  // the order launch's protection bit
+    sl[k] &= 0x7fffu;
+    frm[k] = __ballot(fr[k]);
+    if (lane == 0) wfree[k * SWAVES + wave] = static_cast<int32_t>(__popcll(frm[k]));
+  }
   __syncthreads();
   const int64_t tot_miss = s_tot[2];
   const int32_t lo = static_cast<int32_t>(s_tot[6]), hi = static_cast<int32_t>(s_tot[7]);
@@ -1109,46 +1142,34 @@ __global__ __launch_bounds__(ST) void resolve_split_place_kernel(ResolveBatch ba
   }
   // miss prefix of the workgroup's words
   {
-    int32_t cnt = a0 < a1 ? __popc(first_miss) : 0;
-    for (int64_t wd = a0 + 1; wd < a1; ++wd) cnt += __popc(w.missbits[wd]);
-    int32_t all;
-    int64_t r = s_tot[4] + block_exclusive_sum<int32_t>(cnt, scan32, &all);
+    int64_t r = s_tot[4] + cnt_inc - cnt;
+#pragma unroll
+    for (int u = 0; u < SWAVES; ++u) r += u < wave ? wmiss[u] : 0;
     for (int64_t wd = a0; wd < a1; ++wd) {
       w.mprefix[wd] = static_cast<int32_t>(r);
       r += __popc(wd == a0 ? first_miss : w.missbits[wd]);
     }
   }
   // victims and the new LRU over the workgroup's LRU entries, in LRU order
-  const int32_t S = g.S;
   const int32_t U = static_cast<int32_t>(s_tot[3]);
   const int32_t tm = tot_miss < S ? static_cast<int32_t>(tot_miss) : S;  // only rank < tm matters
   const int32_t Pn = S - U;
   const int32_t fillU = U < tm ? U : tm;
   const int32_t fillP = tm - U > 0 ? (tm - U < Pn ? tm - U : Pn) : 0;
   const int32_t start1 = U - fillU, start2 = U, start3 = S - fillP;
-  Regs<bool, SPLIT_SLOTS> fr;
-#pragma unroll
-  for (int k = 0; k < SPLIT_SLOTS; ++k) {
-    const int64_t j = e0 + T + static_cast<int64_t>(k) * ST;
-    const uint32_t pw = x.prot[(sl[k] < static_cast<uint32_t>(S) ? sl[k] : 0u) >> 5];
-    fr[k] = j < e1 && !((pw >> (sl[k] & 31)) & 1u);
-  }
   int32_t r = static_cast<int32_t>(s_tot[5]);  // unprotected entries before the chunk
 #pragma unroll
   for (int k = 0; k < SPLIT_SLOTS; ++k) {
     const int64_t j = e0 + T + static_cast<int64_t>(k) * ST;
-    const uint64_t m = __ballot(fr[k]);
-    if (lane == 0) wcnt[wave] = static_cast<int32_t>(__popcll(m));
-    __syncthreads();
     int32_t before = 0, chunk = 0;
-    for (int u = 0; u < ST / 64; ++u) {
-      const int32_t c = wcnt[u];
+#pragma unroll
+    for (int u = 0; u < SWAVES; ++u) {
+      const int32_t c = wfree[k * SWAVES + u];
       before += u < wave ? c : 0;
       chunk += c;
     }
-    __syncthreads();
     if (j < e1) {
-      const int32_t rr = r + before + lanes_below(m);  // unprotected entries before entry j
+      const int32_t rr = r + before + lanes_below(frm[k]);  // unprotected entries before entry j
       int32_t rank, at;
       if (fr[k]) {
         rank = rr;
@@ -1395,7 +1416,7 @@ static int resolve_launch(const hs_resolve_desc* descs, int32_t count, char* wor
     const size_t lds = static_cast<size_t>(front_lds);
     const bool l16 = batch.d[0].lru_i16 != 0;  // the same for every descriptor (validated)
     // The split front where it measured faster: hot regions above 16384 rows or histories
-    // above 40000 tokens (7B layer shape, 32768 rows and 131072 tokens: 30.4 us for its three
+    // above 40000 tokens (7B layer shape, 32768 rows and 131072 tokens: 21.9 us for its three
     // launches against 37.5 us for the one-workgroup front; 32B stress shape, 2048 rows and
     // 65536 tokens: the resolve stage 4.20 -> 3.47 ms per step; 0.5B layer shape, 13504 rows
     // and 32768 tokens: 21.7 against 19.3 us, so it keeps the one-workgroup front).
