@@ -439,10 +439,11 @@ static int run_gemm(const void* x, int64_t x_stride, const void* weight, int64_t
   a.out_stride = out_stride;
   a.splits = p.splits;
   a.slice_steps = p.slice_steps;
-  // the split-K partials merged in-kernel unless HS_GEMM_FUSED_MERGE=0 (read per call)
-  const char* fused_env = getenv("HS_GEMM_FUSED_MERGE");
-  const bool fused = !(fused_env && atoi(fused_env) == 0);
+  bool fused = true;
   if (p.splits > 1) {
+    // the split-K partials merged in-kernel unless HS_GEMM_FUSED_MERGE=0 (read per call)
+    const char* fused_env = getenv("HS_GEMM_FUSED_MERGE");
+    fused = !(fused_env && atoi(fused_env) == 0);
     const int64_t need = fused ? p.splits * rows * n * 8 + p.blocks * 8 : p.splits * rows * n * 4;
     HS_CHECK_ARG(workspace != nullptr && workspace_bytes >= need && (reinterpret_cast<uintptr_t>(workspace) & 7) == 0,
                  "GEMM workspace too small or misaligned: need %lld bytes", static_cast<long long>(need));

@@ -11,6 +11,7 @@ for callers that inspect it.
 
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass
 from math import ceil
 
@@ -222,14 +223,10 @@ def quest_topk(queries, minimums, maximums, lengths, page_size, top_pages, keep_
 
 
 def ctypes_void_p_array(n):
-    import ctypes
-
     return ctypes.c_void_p * n
 
 
 def _c_int64_array(n):
-    import ctypes
-
     return ctypes.c_int64 * n
 
 
@@ -257,7 +254,7 @@ def build_union(pages, lengths, page_size, kv_heads, top_pages, keep_sink=True, 
     ecol = torch.empty((batch, kv_heads, entry_cap), dtype=torch.int32, device=device)
     emask = torch.empty((batch, kv_heads, entry_cap), dtype=torch.int32, device=device)
     ecount = torch.empty((batch, kv_heads), dtype=torch.int32, device=device)
-    status = torch.zeros(1, dtype=torch.int32, device=device)
+    status = torch.empty(1, dtype=torch.int32, device=device)  # or-ed into and not read: nothing clears it
     length_arr = (_c_int64_array(batch))(*lengths)
     rc = _lib.load().hs_build_union(
         pages.data_ptr(), pages.stride(0), top, length_arr, page_size, batch, heads, kv_heads,
