@@ -855,9 +855,10 @@ __global__ __launch_bounds__(UT) void build_union_kernel(UnionArgs a) {
   const int64_t b = blockIdx.y;
   const int32_t T = threadIdx.x;
   const int32_t L = static_cast<int32_t>(a.length[b]), P = static_cast<int32_t>(a.P);
-  const int32_t Hq = static_cast<int32_t>(a.Hq), g = static_cast<int32_t>(a.g), top = static_cast<int32_t>(a.top);
+  const int32_t Hq = static_cast<int32_t>(a.Hq), g = static_cast<int32_t>(a.g);
+  const int64_t top = a.top;  // the pages' row stride; it and the capacities may pass 31 bits
   const int32_t count = (L - 1) / P + 1;
-  const int32_t k = top < count ? top : count;
+  const int32_t k = top < count ? static_cast<int32_t>(top) : count;
   const int32_t tail_len = L - (count - 1) * P;
   const int32_t words = (count + 31) / 32;
   const int32_t* pg = a.pages + b * a.p_sb;
@@ -897,67 +898,66 @@ __global__ __launch_bounds__(UT) void build_union_kernel(UnionArgs a) {
 
   if (position) {
     const int32_t upages = rank_of(ubits, uprefix, count - 1) + 1;  // the tail page is always selected
-    const int32_t n = upages * P - (P - tail_len);
-    const int32_t cap = static_cast<int32_t>(a.pos_cap);
+    const int32_t n = (upages - 1) * P + tail_len;
     if (chunk == 0) {
       if (T == 0) {
         a.union_count[b] = n;
-        if (n > cap) atomicOr(a.status, 1);
+        if (n > a.pos_cap) atomicOr(a.status, 1);
       }
       if (a.page_bits)
         for (int32_t w = T; w < words; w += UT) a.page_bits[b * a.pb_stride + w] = ubits[w];
     }
-    int32_t* pos = a.positions + b * a.pos_cap;
-    const int32_t i0 = chunk * UCHUNK, i1 = cap - i0 < UCHUNK ? cap : i0 + UCHUNK;
-    const int32_t nw = n < i1 ? n : i1;
+    // the chunk: `size` positions from c0, the first `held` of them union positions
+    const int64_t c0 = static_cast<int64_t>(chunk) * UCHUNK;
+    int32_t* pos = a.positions + b * a.pos_cap + c0;
+    const int32_t size = a.pos_cap - c0 < UCHUNK ? static_cast<int32_t>(a.pos_cap - c0) : UCHUNK;
+    const int32_t held = n <= c0 ? 0 : n - c0 < size ? static_cast<int32_t>(n - c0) : size;
+    const int32_t i0 = static_cast<int32_t>(c0);  // used where held > 0: below n
     if (a.use_map) {
       for (int32_t p = T; p < count; p += UT)
         if ((ubits[p >> 5] >> (p & 31)) & 1u) rank_page[rank_of(ubits, uprefix, p)] = p;
       __syncthreads();
       // position i: token i % P of the (i / P)-th union page (the tail page is the last)
-      for (int32_t i = i0 + T; i < nw; i += UT) {
-        const int32_t r = page_of(i);
-        pos[i] = rank_page[r] * P + (i - r * P);
+      for (int32_t i = T; i < held; i += UT) {
+        const int32_t r = page_of(i0 + i);
+        pos[i] = rank_page[r] * P + (i0 + i - r * P);
       }
     } else {
       for (int32_t p = T; p < count; p += UT) {
         if (!((ubits[p >> 5] >> (p & 31)) & 1u)) continue;
         const int32_t base = rank_of(ubits, uprefix, p) * P;
         const int32_t plen = p == count - 1 ? tail_len : P;
-        for (int32_t off = 0; off < plen; ++off)
-          if (base + off >= i0 && base + off < i1) pos[base + off] = p * P + off;
+        for (int32_t off = 0; off < plen; ++off) {
+          const int64_t i = base + off - c0;
+          if (i >= 0 && i < held) pos[i] = p * P + off;
+        }
       }
     }
-    for (int32_t i = (n > i0 ? n : i0) + T; i < i1; i += UT) pos[i] = -1;
+    for (int32_t i = held + T; i < size; i += UT) pos[i] = -1;
   } else if (!group) {
     // union columns of the chunk's heads: a head's j-th token (its pages ascending, tail last)
-    const int32_t width = static_cast<int32_t>(a.width);
     const int32_t W = (k - 1) * P + tail_len;
     for (int32_t h = chunk * a.part_heads; h < (chunk + 1) * a.part_heads && h < Hq; ++h) {
       int64_t* hc = a.head_columns + (b * a.Hq + h) * a.width;
       const int32_t* row = pg + h * top;
-      for (int32_t jj = T; jj < width; jj += UT) {
-        int64_t col = -1;
-        if (jj < W) {
-          const int32_t j = page_of(jj);
-          const int32_t p = j < k - 1 ? row[j] : count - 1;
-          col = rank_of(ubits, uprefix, p) * P + (jj - j * P);
-        }
-        hc[jj] = col;
+      for (int32_t jj = T; jj < W; jj += UT) {
+        const int32_t j = page_of(jj);
+        const int32_t p = j < k - 1 ? row[j] : count - 1;
+        hc[jj] = rank_of(ubits, uprefix, p) * P + (jj - j * P);
       }
+      for (int64_t jj = static_cast<int64_t>(W) + T; jj < a.width; jj += UT) hc[jj] = -1;
     }
   } else {
     const int32_t gpages = rank_of(gbits, gprefix, count - 1) + 1;
-    const int32_t E = gpages * P - (P - tail_len);
-    const int32_t cap = static_cast<int32_t>(a.ecap);
-    const int32_t held = E < cap ? E : cap;
+    const int32_t E = (gpages - 1) * P + tail_len;
+    const int32_t held = E < a.ecap ? E : static_cast<int32_t>(a.ecap);
     if (chunk == 0 && T == 0) {
       a.ecount[b * a.Hkv + kv] = held;
-      if (E > cap) atomicOr(a.status, 2);
+      if (E > a.ecap) atomicOr(a.status, 2);
       if (a.estats) atomicAdd(a.estats, static_cast<unsigned long long>(held));
     }
+    if (static_cast<int64_t>(chunk) * UCHUNK >= held) return;
     const int32_t i0 = chunk * UCHUNK, i1 = held - i0 < UCHUNK ? held : i0 + UCHUNK;
-    if (i0 >= held) return;
     if (masks_in_lds) {
       // head bits of each group page, indexed by the page's rank in the group
       for (int32_t i = T; i < g * k; i += UT) {
@@ -1180,7 +1180,8 @@ static int build_union_chunk(const int32_t* pages, int64_t p_stride_b, int64_t t
                  static_cast<long long>(width), static_cast<long long>(W));
     a.length[i] = lengths[i];
   }
-  a.P = page_size;
+  // a page of more tokens than the longest history holds what one of that many does
+  a.P = std::min(page_size, *std::max_element(lengths, lengths + batch));
   a.Hq = heads;
   a.Hkv = kv_heads;
   a.g = heads / kv_heads;
@@ -1210,7 +1211,7 @@ static int build_union_chunk(const int32_t* pages, int64_t p_stride_b, int64_t t
     (void)hipGetLastError();
     lds_attr = true;
   }
-  a.pshift = (page_size & (page_size - 1)) == 0 ? __builtin_ctzll(static_cast<unsigned long long>(page_size)) : -1;
+  a.pshift = (a.P & (a.P - 1)) == 0 ? __builtin_ctzll(static_cast<unsigned long long>(a.P)) : -1;
   a.pos_parts = static_cast<int>(ceil_div(pos_capacity, UCHUNK));
   a.entry_parts = static_cast<int>(ceil_div(entry_capacity, UCHUNK));
   a.part_heads = static_cast<int>(std::max<int64_t>(1, UCHUNK / width));
@@ -1277,6 +1278,7 @@ extern "C" int hs_build_union(const int32_t* pages, int64_t p_stride_b, int64_t 
   HS_CHECK_ARG(heads >= 1 && kv_heads >= 1 && heads % kv_heads == 0, "invalid GQA shape");
   for (int64_t i = 0; i < batch; ++i) {  // every request, before the first launch
     HS_CHECK_ARG(lengths[i] >= 1, "cannot build a union over an empty history");
+    HS_CHECK_ARG(lengths[i] <= INT32_MAX, "union positions are 32-bit: %lld tokens", static_cast<long long>(lengths[i]));
     HS_CHECK_ARG(ceil_div(lengths[i], page_size) <= UMAXPAGES, "too many pages for the union builder");
     const int64_t count = ceil_div(lengths[i], page_size);
     const int64_t k = top < count ? top : count;

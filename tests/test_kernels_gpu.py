@@ -518,6 +518,31 @@ def test_union_builder_chunk_edges(gpu, pages, P, kv, g, top, length):
     test_union_builder_matches_host_adapter(gpu, pages, P, kv, g, top, length)
 
 
+@pytest.mark.parametrize("top,P,length", [(2**32 + 1, 16, 40), (3, 2**33, 5), (2**32, 2**32 + 1, 7)])
+def test_union_builder_sizes_past_31_bits(gpu, top, P, length):
+    """A page budget and a page size of more than 31 bits: the whole history."""
+    from mini_hisparse_amd import _lib
+
+    count = -(-length // P)
+    pages = torch.arange(count, dtype=torch.int32, device=gpu)
+    pos, columns = torch.empty(64, dtype=torch.int32, device=gpu), torch.empty(64, dtype=torch.int64, device=gpu)
+    ecol, emask, counts = (torch.zeros(n, dtype=torch.int32, device=gpu) for n in (64, 64, 3))
+
+    def build(tokens):
+        return _lib.load().hs_build_union(
+            pages.data_ptr(), top, top, (ctypes.c_int64 * 1)(tokens), P, 1, 1, 1, pos.data_ptr(), 64,
+            columns.data_ptr(), 64, counts.data_ptr(), ecol.data_ptr(), emask.data_ptr(), 64, counts[1:].data_ptr(),
+            counts[2:].data_ptr(), None, 0, None, _lib.stream_handle(gpu))
+
+    _lib.check(build(length), "hs_build_union")
+    expected = torch.cat([torch.arange(length), torch.full((64 - length,), -1)])
+    assert torch.equal(pos.cpu().long(), expected) and torch.equal(columns.cpu(), expected)
+    assert torch.equal(ecol[:length].cpu().long(), expected[:length]) and bool((emask[:length] == 1).all())
+    assert counts.tolist() == [length, length, 0]
+    if P > 2**31:  # one page of more tokens than a position can number
+        assert build(2**31) != 0
+
+
 # --------------------------------------------------------------------- gather
 # rows of 2 KB and 1 KB (one row plane per wave instruction), 256, 128 and 8 bytes (a wave
 # instruction reads one plane of 4, 8 and 64 consecutive entries), 32 bytes (2 units) and 96
