@@ -6,7 +6,7 @@
 // 16 weight rows as the MFMA's M dimension and the (padded) token rows as its
 // N dimension, so the MFMA's output tile is 16 weight rows x 16 tokens.
 //
-// A workgroup (4 or 8 waves) owns 16 or 32 weight rows and one K slice; wave w
+// A workgroup (4 or 8 waves) owns 16 to 32 weight rows and one K slice; wave w
 // takes k-steps (of 32) in groups of GU consecutive steps, round-robin over
 // the waves, so within a round the waves read GU * 64 contiguous bytes of every
 // row each.  Per round a lane issues all of its loads (GU weight fragments of
@@ -52,6 +52,7 @@ struct GemmArgs {
   int64_t out_stride;
   float* part;  // [splits, M, N] when splits > 1
   int64_t splits, slice_steps;
+  int64_t rows;  // WINDOW: weight rows of a workgroup
   int64_t F;  // SWIGLU: output features (N = 2 * 16 * ceil(F / 16) interleaved weight rows)
   unsigned long long* keys;  // ARGMAX: [M, gridDim.x] best key per token and workgroup
   // split-K merged in-kernel (epoch != 0): tagged partial words [splits, M, N] and one
@@ -94,25 +95,39 @@ __device__ __forceinline__ float gemm_round(float v) {
 // SiLU rounded, then the product (hs_silu_mul).
 // ARGMAX (one K slice): per token the workgroup's best key over its rows, each
 // logit rounded to the dtype after the bias as the plain form stores it.
-template <int DT, int GM_TILES, int NW, bool TILED, bool NT, bool SWIGLU = false, bool ARGMAX = false>
+// WINDOW: the workgroup's a.rows weight rows start anywhere in its first tile (plan_gemm).
+template <int DT, int GM_TILES, int NW, bool TILED, bool NT, bool SWIGLU = false, bool ARGMAX = false, bool WINDOW = false>
 __global__ __launch_bounds__(64 * NW) void skinny_gemm_kernel(GemmArgs a) {
   constexpr int GU = 8;  // k-steps of a wave's round
   constexpr int GM_T = 64 * NW;
-  constexpr int GM_ROWS = 16 * GM_TILES;  // weight rows per workgroup
+  constexpr int GM_ROWS = 16 * GM_TILES;  // weight rows of the workgroup's tiles
   __shared__ float red[NW][GM_ROWS][17];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c = lane & 15, j = lane >> 4;
-  const int64_t n0 = static_cast<int64_t>(blockIdx.x) * GM_ROWS;
+  // weight rows n0 .. n1, in the tiles from nb
+  const int64_t n0 = static_cast<int64_t>(blockIdx.x) * (WINDOW ? a.rows : GM_ROWS);
+  const int64_t nb = WINDOW ? n0 & ~static_cast<int64_t>(15) : n0;
+  const int64_t n1 = WINDOW && n0 + a.rows < a.N ? n0 + a.rows : a.N;
+  auto dropped = [&](int64_t n) -> bool { return n >= n1 || (WINDOW && n < n0); };
   const int64_t split = blockIdx.y;
   const int64_t steps = a.K / 32;
   const int64_t s0 = split * a.slice_steps;
   int64_t s1 = s0 + a.slice_steps;
   if (s1 > steps) s1 = steps;
-  // lane (c, j): weight rows n0 + 16t + c, token row c, k offset 8j within a step
+  // lane (c, j): weight rows nb + 16t + c, token row c, k offset 8j within a step
   const unsigned short* wrow[GM_TILES];
 #pragma unroll
   for (int t = 0; t < GM_TILES; ++t) {
-    if constexpr (TILED) {
+    if constexpr (WINDOW) {
+      // a lane outside the rows reads the first or the last one again, a tile past them the
+      // last tile (no more bytes of the weight); their outputs are dropped
+      const int64_t last = (n1 - 1) >> 4;
+      const int64_t nt = (nb >> 4) + t < last ? (nb >> 4) + t : last;
+      const int lo = n0 > 16 * nt ? static_cast<int>(n0 - 16 * nt) : 0;
+      const int hi = n1 - 1 - 16 * nt < 15 ? static_cast<int>(n1 - 1 - 16 * nt) : 15;
+      const int row = c < lo ? lo : c > hi ? hi : c;
+      wrow[t] = TILED ? a.w + nt * steps * 512 + row * 32 + 8 * j : a.w + (16 * nt + row) * a.K + 8 * j;
+    } else if constexpr (TILED) {
       const int64_t tiles = (a.N + 15) / 16;
       int64_t nt = n0 / 16 + t;
       if (nt >= tiles) nt = tiles - 1;  // tiles past N read the last one; their outputs are dropped
@@ -186,9 +201,9 @@ __global__ __launch_bounds__(64 * NW) void skinny_gemm_kernel(GemmArgs a) {
     __shared__ unsigned long long best[GM_ROWS][16];
     for (int idx = threadIdx.x; idx < GM_ROWS * 16; idx += GM_T) {
       const int r = idx >> 4, m = idx & 15;
-      const int64_t n = n0 + r;
+      const int64_t n = nb + r;
       unsigned long long key = 0;
-      if (n < a.N) {
+      if (!dropped(n)) {
         const float b = a.bias != nullptr ? load_elem<DT>(a.bias, n) : 0.f;
         key = argmax_key(gemm_round<DT>(sum_of(r, m) + b), n);
       }
@@ -211,8 +226,8 @@ __global__ __launch_bounds__(64 * NW) void skinny_gemm_kernel(GemmArgs a) {
     const uint32_t tag = group_tag(a.epoch, round);
     for (int idx = threadIdx.x; idx < GM_ROWS * 16; idx += GM_T) {
       const int r = idx >> 4, m = idx & 15;
-      const int64_t n = n0 + r;
-      if (m >= a.M || n >= a.N) continue;
+      const int64_t n = nb + r;
+      if (m >= a.M || dropped(n)) continue;
       store_partial(a.words + (split * a.M + m) * a.N + n, sum_of(r, m), tag);
     }
     __shared__ int s_last;
@@ -224,8 +239,8 @@ __global__ __launch_bounds__(64 * NW) void skinny_gemm_kernel(GemmArgs a) {
     const int64_t sstride = a.M * a.N;
     for (int idx = threadIdx.x; idx < GM_ROWS * 16; idx += GM_T) {
       const int r = idx >> 4, m = idx & 15;
-      const int64_t n = n0 + r;
-      if (m >= a.M || n >= a.N) continue;
+      const int64_t n = nb + r;
+      if (m >= a.M || dropped(n)) continue;
       const unsigned long long* w0 = a.words + m * a.N + n;
       float v = 0.f;
       for (int64_t s0 = 0; s0 < a.splits; s0 += MS) {
@@ -254,8 +269,8 @@ __global__ __launch_bounds__(64 * NW) void skinny_gemm_kernel(GemmArgs a) {
   }
   for (int idx = threadIdx.x; idx < GM_ROWS * 16; idx += GM_T) {
     const int r = idx >> 4, m = idx & 15;
-    const int64_t n = n0 + r;
-    if (m >= a.M || n >= a.N) continue;
+    const int64_t n = nb + r;
+    if (m >= a.M || dropped(n)) continue;
     const float v = sum_of(r, m);
     if (a.splits > 1) {
       a.part[(split * a.M + m) * a.N + n] = v;
@@ -316,6 +331,7 @@ __global__ __launch_bounds__(FIN_T) void argmax_finalize_kernel(const unsigned l
 struct GemmPlan {
   int tiles, waves;
   bool stream;  // non-temporal weight loads
+  int64_t rows;  // weight rows per workgroup where they cross tile edges, else 0
   int64_t blocks, splits, slice_steps;
 };
 
@@ -335,10 +351,9 @@ static int gemm_waves(int64_t N, int64_t slice_steps) { return slice_steps > 32 
 // (1 KB each), an eighth more with one tile, which reads x twice as often per weight byte.
 // Merging K slices costs about 48 tile-steps (2 us), and pays only within one round or for
 // long slices.  Measured, 8 rows, us before (at least 512 workgroups of 4 waves) and with
-// these plans: 4608 x 3584 12.6 and 12.0, 3584 x 18944 34.2 and 29.6 (two tiles in two slices
-// instead of one in three), 7168 x 5120 21.6 and 15.7, 5120 x 5120 17.2 and 15.6 (two tiles),
-// 5120 x 27648 64.9 and 53.3 (two tiles in three slices), 896 x 4864 9.6 and 7.5 (three
-// slices), 3584 x 3584 9.9 and 8.1.
+// these plans: 3584 x 18944 34.2 and 29.6 (two tiles in two slices instead of one in three),
+// 7168 x 5120 21.6 and 15.7, 5120 x 27648 64.9 and 53.3 (two tiles in three slices),
+// 896 x 4864 9.6 and 7.5 (three slices), 3584 x 3584 9.9 and 8.1.
 static GemmPlan plan_gemm(int64_t N, int64_t K, bool one_slice = false) {
   // unsigned, with constant divisors: every projection call plans, on the host's time
   constexpr uint64_t CUS = 256, X_SHARE = 8, MERGE = 48, LONG_SLICE = 256;
@@ -363,6 +378,22 @@ static GemmPlan plan_gemm(int64_t N, int64_t K, bool one_slice = false) {
       p.slice_steps = static_cast<int64_t>(slice);
     }
   }
+  // Where two tiles per workgroup leave CUs idle (4096 < N <= 6144), the rows are dealt evenly
+  // instead: an even count (two are a 128-byte line of a k-step) of 18, 20 or 24, which two
+  // tiles hold wherever it starts.  us, two whole tiles and this, 8 rows (16 rows): 4608 x 3584
+  // 12.2 and 10.3 (14.2 and 12.2), 5120 x 5120 15.9 and 13.6 (19.2 and 16.9), 6144 x 4096 13.2
+  // and 12.6 (15.9 and 14.5).  Fewer rows than a tile's, or two rounds, do not pay: the second
+  // tile's loads cost more than the bytes they leave out (3584 x 3584 in one tile 8.0, in
+  // 14 rows of two 9.7; 9216 x 4096 19.0 and 20.7).  Longer K stays in slices.
+  uint64_t rows = 2 * ((static_cast<uint64_t>(N) + 2 * CUS - 1) / (2 * CUS));
+  if (rows == 22) rows = 24;  // starts at multiples of 2: 22 rows could touch a third tile
+  if (!one_slice && rows > 16 && rows <= 24 && steps <= 2 * LONG_SLICE && steps * rows / 16 < best) {
+    p.tiles = 2;
+    p.rows = static_cast<int64_t>(rows);
+    p.blocks = gemm_ceil(N, p.rows);
+    p.splits = 1;
+    p.slice_steps = static_cast<int64_t>(steps);
+  }
   p.waves = gemm_waves(N, p.slice_steps);
   // A weight is read once per step.  Above the 4 MB of an XCD's L2 nothing of it is left
   // for the next step, and keeping it costs: 2 x 18944 x 3584 52.4 us, non-temporal 48.2;
@@ -380,6 +411,13 @@ static void launch_gemm_waves(const GemmPlan& p, dim3 grid, const GemmArgs& a, h
 
 template <int DT, bool TILED, bool NT, bool ARGMAX>
 static void launch_gemm_tiles(const GemmPlan& p, dim3 grid, const GemmArgs& a, hipStream_t s) {
+  if constexpr (!ARGMAX) {
+    if (p.rows > 0) {
+      if (p.waves == 8) hipLaunchKernelGGL((skinny_gemm_kernel<DT, 2, 8, TILED, NT, false, false, true>), grid, dim3(512), 0, s, a);
+      else hipLaunchKernelGGL((skinny_gemm_kernel<DT, 2, 4, TILED, NT, false, false, true>), grid, dim3(256), 0, s, a);
+      return;
+    }
+  }
   if (p.tiles == 1) launch_gemm_waves<DT, 1, TILED, NT, ARGMAX>(p, grid, a, s);
   else launch_gemm_waves<DT, 2, TILED, NT, ARGMAX>(p, grid, a, s);
 }
@@ -438,6 +476,7 @@ static int run_gemm(const void* x, int64_t x_stride, const void* weight, int64_t
   a.out = out;
   a.out_stride = out_stride;
   a.splits = p.splits;
+  a.rows = p.rows;
   a.slice_steps = p.slice_steps;
   bool fused = true;
   if (p.splits > 1) {

@@ -356,6 +356,21 @@ def test_projection_plans_at_their_edges(gpu, rows, n, k):
     assert torch.equal(linear_swiglu_tiled(x, tile_gate_up(w, n // 2), n // 2), silu_mul(y))
 
 
+# row counts whose workgroups take 18, 20 or 24 weight rows wherever these start in the 16-row
+# tiles, the counts beside them (a last workgroup of one row, a full one), and K at the
+# longest that does so and one step past it
+WINDOW_SHAPES = [(4096, 64), (4097, 1056), (4608, 64), (4609, 64), (5120, 1024), (5121, 64), (5632, 64), (5640, 1056),
+                 (6144, 64), (6145, 64), (4608, 16384), (4608, 16416)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 16])
+@pytest.mark.parametrize("n,k", WINDOW_SHAPES)
+def test_projection_rows_across_tile_edges(gpu, rows, n, k):
+    """Workgroups whose rows start inside a tile, with the bias, row-major and tiled."""
+    test_linear_matches_an_fp32_reference(gpu, torch.bfloat16, rows, n, k, True)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("n", [16, 32800, 262144, 262176])
 def test_argmax_key_counts(gpu, n):
