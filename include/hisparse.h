@@ -122,7 +122,8 @@ int hs_uniform_pages(uint64_t seed, uint64_t step, const int64_t* page_counts, i
  * Replaces: Selection.from_pages (selection.py:43-60) followed by
  * LogicalTopK.from_selection (row_index.py:20-31), without the host sync of
  * selection.py:100.
- *   pages         [batch, heads, top] from hs_quest_topk; lengths host [batch]
+ *   pages         [batch, heads, top] from hs_quest_topk; lengths host [batch], each at
+ *                 most 2^31 - 1 (positions are 32-bit)
  *   positions     [batch, pos_capacity] int32: ascending union of the
  *                 selected tokens, then -1
  *   head_columns  [batch, heads, width] int64: union column of each head's
