@@ -796,7 +796,7 @@ struct UnionArgs {
   int64_t maxcount;      // pages of the longest history
   int use_map;           // rank -> page map in LDS (maxcount <= UMAPPAGES)
   int pshift;            // log2 P, or -1
-  int pos_parts, entry_parts, part_heads;  // workgroups of the positions, of a KV head's entries; heads of a workgroup
+  int parts, pos_parts, entry_parts, part_heads;  // workgroups in all, of the positions, of a KV head's entries; heads of a workgroup
 };
 
 __device__ __forceinline__ bool head_has_page(const int32_t* row, int64_t k, int32_t p) {
@@ -826,6 +826,8 @@ __device__ __forceinline__ bool head_has_page(const int32_t* row, int64_t k, int
 constexpr int64_t UMAXMASK = 4096;  // group pages (g * top) with an LDS mask slot
 constexpr int64_t UMAPPAGES = 24576;  // longest history (pages) with an LDS rank -> page map
 constexpr int32_t UCHUNK = 4096;
+constexpr int64_t UGRID = 1 << 20;  // workgroups of one grid row: the next ones are in the third dimension
+constexpr int64_t UMAXHEADS = 1 << 22;
 
 // prefix[w] = set bits of bits[0 .. w), by one wave; returns all set bits.
 __device__ __forceinline__ void prefix_popcounts(const uint32_t* bits, uint32_t* prefix, int32_t words) {
@@ -863,7 +865,8 @@ __global__ __launch_bounds__(UT) void build_union_kernel(UnionArgs a) {
   const int32_t words = (count + 31) / 32;
   const int32_t* pg = a.pages + b * a.p_sb;
   // the role and its chunk
-  int32_t part = blockIdx.x;
+  int32_t part = static_cast<int32_t>(blockIdx.z * gridDim.x + blockIdx.x);
+  if (part >= a.parts) return;
   const bool position = part < a.pos_parts;
   if (!position) part -= a.pos_parts;
   const bool group = !position && part < static_cast<int32_t>(a.Hkv) * a.entry_parts;
@@ -872,7 +875,7 @@ __global__ __launch_bounds__(UT) void build_union_kernel(UnionArgs a) {
   const int32_t chunk = group ? part - kv * a.entry_parts : part;
   const bool masks_in_lds = g * k <= UMAXMASK;
   // page and row of a token offset: a shift where the page size is a power of two
-  auto page_of = [&](int32_t i) { return a.pshift >= 0 ? i >> a.pshift : static_cast<int32_t>(static_cast<uint32_t>(i) / static_cast<uint32_t>(P)); };
+  auto page_of = [&](uint32_t i) { return static_cast<int32_t>(a.pshift >= 0 ? i >> a.pshift : i / static_cast<uint32_t>(P)); };
 
   for (int32_t i = T; i < words; i += UT) {
     ubits[i] = 0u;
@@ -881,12 +884,20 @@ __global__ __launch_bounds__(UT) void build_union_kernel(UnionArgs a) {
   if (group && masks_in_lds)
     for (int32_t i = T; i < g * k; i += UT) gmask[i] = 0u;
   __syncthreads();
-  for (int32_t i = T; i < Hq * k; i += UT) {
-    const int32_t h = i / k;
-    const int32_t p = pg[h * top + (i - h * k)];
-    if (p < 0 || p >= count) continue;
-    atomicOr(&ubits[p >> 5], 1u << (p & 31));
-    if (group && h / g == kv) atomicOr(&gbits[p >> 5], 1u << (p & 31));
+  // the thread's pages, UT apart; heads times pages may pass 31 bits, so head and page are stepped
+  const int32_t step_h = UT / k, step_j = UT - step_h * k;
+  for (int32_t h = T / k, j = T - h * k; h < Hq;) {
+    const int32_t p = pg[h * top + j];
+    if (p >= 0 && p < count) {
+      atomicOr(&ubits[p >> 5], 1u << (p & 31));
+      if (group && h / g == kv) atomicOr(&gbits[p >> 5], 1u << (p & 31));
+    }
+    h += step_h;
+    j += step_j;
+    if (j >= k) {
+      j -= k;
+      ++h;
+    }
   }
   __syncthreads();
   if (T < 64) prefix_popcounts(ubits, uprefix, words);
@@ -940,10 +951,11 @@ __global__ __launch_bounds__(UT) void build_union_kernel(UnionArgs a) {
     for (int32_t h = chunk * a.part_heads; h < (chunk + 1) * a.part_heads && h < Hq; ++h) {
       int64_t* hc = a.head_columns + (b * a.Hq + h) * a.width;
       const int32_t* row = pg + h * top;
-      for (int32_t jj = T; jj < W; jj += UT) {
+      // unsigned: the step past the last column of a history of 2^31 - 1 tokens passes 31 bits
+      for (uint32_t jj = T; jj < static_cast<uint32_t>(W); jj += UT) {
         const int32_t j = page_of(jj);
         const int32_t p = j < k - 1 ? row[j] : count - 1;
-        hc[jj] = rank_of(ubits, uprefix, p) * P + (jj - j * P);
+        hc[jj] = rank_of(ubits, uprefix, p) * P + (static_cast<int32_t>(jj) - j * P);
       }
       for (int64_t jj = static_cast<int64_t>(W) + T; jj < a.width; jj += UT) hc[jj] = -1;
     }
@@ -957,7 +969,8 @@ __global__ __launch_bounds__(UT) void build_union_kernel(UnionArgs a) {
       if (a.estats) atomicAdd(a.estats, static_cast<unsigned long long>(held));
     }
     if (static_cast<int64_t>(chunk) * UCHUNK >= held) return;
-    const int32_t i0 = chunk * UCHUNK, i1 = held - i0 < UCHUNK ? held : i0 + UCHUNK;
+    const uint32_t i0 = static_cast<uint32_t>(chunk) * UCHUNK;  // below held; the step past i1 may pass 31 bits
+    const uint32_t i1 = static_cast<uint32_t>(held) - i0 < UCHUNK ? static_cast<uint32_t>(held) : i0 + UCHUNK;
     if (masks_in_lds) {
       // head bits of each group page, indexed by the page's rank in the group
       for (int32_t i = T; i < g * k; i += UT) {
@@ -974,9 +987,9 @@ __global__ __launch_bounds__(UT) void build_union_kernel(UnionArgs a) {
         if ((gbits[p >> 5] >> (p & 31)) & 1u) rank_page[rank_of(gbits, gprefix, p)] = rank_of(ubits, uprefix, p);
       __syncthreads();
       // entry i: token i % P of the (i / P)-th group page, its union column and head mask
-      for (int32_t i = i0 + T; i < i1; i += UT) {
+      for (uint32_t i = i0 + T; i < i1; i += UT) {
         const int32_t r = page_of(i);
-        ec[i] = rank_page[r] * P + (i - r * P);
+        ec[i] = rank_page[r] * P + (static_cast<int32_t>(i) - r * P);
         em[i] = gmask[r];
       }
       return;
@@ -996,7 +1009,7 @@ __global__ __launch_bounds__(UT) void build_union_kernel(UnionArgs a) {
       const int32_t ubase = rank_of(ubits, uprefix, p) * P;
       const int32_t plen = p == count - 1 ? tail_len : P;
       for (int32_t off = 0; off < plen; ++off) {
-        const int32_t i = gbase + off;
+        const uint32_t i = gbase + off;
         if (i >= i0 && i < i1) {
           ec[i] = ubase + off;
           em[i] = mask;
@@ -1162,6 +1175,7 @@ static int build_union_chunk(const int32_t* pages, int64_t p_stride_b, int64_t t
   HS_CHECK_ARG(top >= 1 && page_size >= 1 && heads >= 1 && kv_heads >= 1 && heads % kv_heads == 0,
                "invalid union shape");
   HS_CHECK_ARG(heads / kv_heads <= 32, "at most 32 query heads per KV head");
+  HS_CHECK_ARG(heads <= UMAXHEADS, "too many query heads for the union builder");
   HS_CHECK_ARG(pages && lengths && positions && head_columns && union_count && entry_columns &&
                    entry_masks && entry_counts && status,
                "null union pointer");
@@ -1212,12 +1226,18 @@ static int build_union_chunk(const int32_t* pages, int64_t p_stride_b, int64_t t
     lds_attr = true;
   }
   a.pshift = (a.P & (a.P - 1)) == 0 ? __builtin_ctzll(static_cast<unsigned long long>(a.P)) : -1;
-  a.pos_parts = static_cast<int>(ceil_div(pos_capacity, UCHUNK));
-  a.entry_parts = static_cast<int>(ceil_div(entry_capacity, UCHUNK));
+  const int64_t pos_parts = ceil_div(pos_capacity, UCHUNK);
+  // a KV head has at most one entry per token
+  const int64_t entry_parts = ceil_div(std::min(entry_capacity, *std::max_element(lengths, lengths + batch)), UCHUNK);
   a.part_heads = static_cast<int>(std::max<int64_t>(1, UCHUNK / width));
-  const int64_t parts = a.pos_parts + kv_heads * a.entry_parts + ceil_div(heads, a.part_heads);
-  hipLaunchKernelGGL(build_union_kernel, dim3(static_cast<unsigned>(parts), static_cast<unsigned>(batch)),
-                     dim3(UT), lds, stream, a);
+  const int64_t parts = pos_parts + kv_heads * entry_parts + ceil_div(heads, a.part_heads);
+  HS_CHECK_ARG(pos_parts <= INT32_MAX / 2 && parts <= INT32_MAX - UGRID, "union capacities too large");
+  a.parts = static_cast<int>(parts);
+  a.pos_parts = static_cast<int>(pos_parts);
+  a.entry_parts = static_cast<int>(entry_parts);
+  const dim3 grid(static_cast<unsigned>(std::min(parts, UGRID)), static_cast<unsigned>(batch),
+                  static_cast<unsigned>(ceil_div(parts, UGRID)));
+  hipLaunchKernelGGL(build_union_kernel, grid, dim3(UT), lds, stream, a);
   HS_CHECK_LAUNCH("union builder");
   return HS_OK;
 }

@@ -543,6 +543,30 @@ def test_union_builder_sizes_past_31_bits(gpu, top, P, length):
         assert build(2**31) != 0
 
 
+@pytest.mark.parametrize("P", [2**30, 2**30 + 3])
+def test_union_builder_of_the_longest_history(gpu, P):
+    """2^31 - 1 tokens, every page selected: the last step of a thread through a head's columns or a
+    KV head's entries passes 31 bits.  Positions past their capacity raise the status."""
+    from mini_hisparse_amd import _lib
+
+    L, cap, part = 2**31 - 1, 64, 2**27
+    if torch.cuda.mem_get_info()[0] < 48 * 2**30:
+        pytest.skip("needs 35 GB of device memory")
+    pages = torch.tensor([0, 1], dtype=torch.int32, device=gpu)
+    pos, counts = torch.empty(cap, dtype=torch.int32, device=gpu), torch.zeros(3, dtype=torch.int32, device=gpu)
+    columns = torch.empty(L, dtype=torch.int64, device=gpu)
+    ecol, emask = (torch.empty(L, dtype=torch.int32, device=gpu) for _ in range(2))
+    _lib.check(_lib.load().hs_build_union(
+        pages.data_ptr(), 2, 2, (ctypes.c_int64 * 1)(L), P, 1, 1, 1, pos.data_ptr(), cap, columns.data_ptr(), L,
+        counts.data_ptr(), ecol.data_ptr(), emask.data_ptr(), L, counts[1:].data_ptr(), counts[2:].data_ptr(), None, 0,
+        None, _lib.stream_handle(gpu)), "hs_build_union")
+    assert counts.tolist() == [L, L, 1] and pos.tolist() == list(range(cap))
+    for c0 in range(0, L, part):
+        expected = torch.arange(c0, min(L, c0 + part), device=gpu)
+        assert torch.equal(columns[c0 : c0 + part], expected) and torch.equal(ecol[c0 : c0 + part].long(), expected)
+        assert bool((emask[c0 : c0 + part] == 1).all())
+
+
 # --------------------------------------------------------------------- gather
 # rows of 2 KB and 1 KB (one row plane per wave instruction), 256, 128 and 8 bytes (a wave
 # instruction reads one plane of 4, 8 and 64 consecutive entries), 32 bytes (2 units) and 96
