@@ -796,7 +796,8 @@ struct UnionArgs {
   int64_t maxcount;      // pages of the longest history
   int use_map;           // rank -> page map in LDS (maxcount <= UMAPPAGES)
   int pshift;            // log2 P, or -1
-  int parts, pos_parts, entry_parts, part_heads;  // workgroups in all, of the positions, of a KV head's entries; heads of a workgroup
+  int chunk, part_heads;  // positions or entries, and heads, of a workgroup
+  int parts, pos_parts, entry_parts;  // workgroups in all, of the positions, of a KV head's entries
 };
 
 __device__ __forceinline__ bool head_has_page(const int32_t* row, int64_t k, int32_t p) {
@@ -809,25 +810,31 @@ __device__ __forceinline__ bool head_has_page(const int32_t* row, int64_t k, int
   return lo < k && row[lo] == p;
 }
 
-// Workgroups of one request (blockIdx.y), by blockIdx.x: UCHUNK union positions each;
-// then, per KV head, UCHUNK of its group entries each; then about UCHUNK union columns of
-// a few query heads each.  Every workgroup rebuilds the selected-page bitmap and its word
-// prefix popcounts in LDS (a few hundred words) from the heads' pages, so none waits for
-// another.  The launch is bound by that chain of steps and by what the longest workgroup
-// writes after it: equal chunks keep the second part short, and indexes are 32-bit with
-// pages of a power of two taken by shifts (a 64-bit division by a runtime page size costs
-// more than the store it serves).  Positions and entries are written one output element
-// per thread through an LDS map from a page's rank to the page, a group entry's head mask
-// comes from an LDS array indexed by the page's rank among the group's pages.
-// Measured (kernel trace, 28 heads x 64 of 8192 pages, 16 requests): 8.9 us, against 19.5
-// us with one workgroup per head, KV head and position list and 64-bit indexes; 512
-// threads with chunks of 2048 10.1 us, 1024 with 2048 14.6 us (more workgroups rebuild the
-// bitmap).  14 heads x 32 of 2048 pages, 4 requests: 6.0 against 6.8 us.
+// Workgroups of one request (blockIdx.y), by blockIdx.x: a chunk of union positions each;
+// then, per KV head, a chunk of its group entries each; then the union columns of up
+// to UCHUNK / UT query heads each, one after the other.  Every workgroup rebuilds the selected-page bitmap and its
+// word prefix popcounts in LDS (a few hundred words) from the heads' pages, so none waits for
+// another; one whose chunk no list of the request reaches ends before that.  The launch is
+// bound by that chain of steps and by what the longest workgroup writes after it: equal
+// chunks keep the second part short, and indexes are 32-bit with pages of a power of two
+// taken by shifts (a 64-bit division by a runtime page size costs more than the store it
+// serves).  Positions and entries are written one output element per thread through an LDS
+// map from a page's rank to the page, a group entry's head mask comes from an LDS array
+// indexed by the page's rank among the group's pages.
+// A chunk is UCHUNK while a CU has one workgroup at most, and doubles up to UCHUNK_MAX while
+// they have more: rebuilding the bitmap then costs more than a chunk's stores.
+// us per launch with one workgroup per head, KV head and position list and 64-bit indexes, with
+// chunks of 4096 and heads of 4096 columns whatever they cost, and now (heads x pages of the
+// history's, requests): 28 x 64 of 8192, 16: 20.0, 9.4 and 8.2; 64 x 4 of 13, 1: 5.8, 17.1 and
+// 4.8; 64 x 512 of 8192, 16: 114, 146 and 78; 64 x 2000 of 4096, 16: 601, 1097 and 480; 64 x 32
+// of 125 with lists for 64 times as many, 16: 26.5, 43.9 and 9.1.
 constexpr int64_t UMAXMASK = 4096;  // group pages (g * top) with an LDS mask slot
 constexpr int64_t UMAPPAGES = 24576;  // longest history (pages) with an LDS rank -> page map
-constexpr int32_t UCHUNK = 4096;
+constexpr int64_t UCHUNK = 4096;
+constexpr int64_t UCHUNK_MAX = 16384;
 constexpr int64_t UGRID = 1 << 20;  // workgroups of one grid row: the next ones are in the third dimension
 constexpr int64_t UMAXHEADS = 1 << 22;
+constexpr int64_t UCUS = 256;
 
 // prefix[w] = set bits of bits[0 .. w), by one wave; returns all set bits.
 __device__ __forceinline__ void prefix_popcounts(const uint32_t* bits, uint32_t* prefix, int32_t words) {
@@ -844,15 +851,38 @@ __device__ __forceinline__ void prefix_popcounts(const uint32_t* bits, uint32_t*
   }
 }
 
+// Both bitmaps' prefixes by the whole workgroup, two words a thread: for more words than a
+// wave should walk.
+__device__ __forceinline__ void block_prefix_popcounts(const uint32_t* ubits, uint32_t* uprefix, const uint32_t* gbits,
+                                                       uint32_t* gprefix, int32_t words, uint64_t* scan) {
+  static_assert(UMAXPAGES <= 2 * 32 * UT, "two words a thread");
+  const int32_t w = 2 * static_cast<int32_t>(threadIdx.x), wave = threadIdx.x >> 6;
+  auto both = [&](int32_t i) -> uint64_t {  // the group's count above the union's
+    return i < words ? static_cast<uint64_t>(__popc(gbits[i])) << 32 | static_cast<uint64_t>(__popc(ubits[i])) : 0u;
+  };
+  const uint64_t c0 = both(w), c1 = both(w + 1);
+  uint64_t at = wave_inclusive_sum(c0 + c1);
+  if ((threadIdx.x & 63) == 63) scan[wave] = at;
+  __syncthreads();
+  at -= c0 + c1;
+  for (int32_t u = 0; u < wave; ++u) at += scan[u];
+  for (int32_t i = w; i < w + 2 && i < words; ++i, at += c0) {
+    uprefix[i] = static_cast<uint32_t>(at);
+    gprefix[i] = static_cast<uint32_t>(at >> 32);
+  }
+}
+
 // Dynamic LDS: four bitmaps of `a.words` words and a rank -> page map of `a.maxcount`
-// entries (longest history of the batch).
-__global__ __launch_bounds__(UT) void build_union_kernel(UnionArgs a) {
+// entries (longest history of the batch).  At most 80 SGPRs: with more a SIMD was seen to hold
+// seven waves, so a CU one workgroup instead of two (16 requests, 64 heads x 512 pages: 78 us with
+// 80, 106 with 81).
+__global__ __launch_bounds__(UT) __attribute__((amdgpu_num_sgpr(80))) void build_union_kernel(UnionArgs a) {
   extern __shared__ uint32_t union_lds[];
   uint32_t* ubits = union_lds;
   uint32_t* uprefix = ubits + a.words;
   uint32_t* gbits = uprefix + a.words;
   uint32_t* gprefix = gbits + a.words;
-  int32_t* rank_page = reinterpret_cast<int32_t*>(gprefix + a.words);  // [maxcount]
+  int32_t* rank_page = reinterpret_cast<int32_t*>(gprefix + a.words);  // [maxcount], or scan scratch [32]
   __shared__ uint32_t gmask[UMAXMASK];
   const int64_t b = blockIdx.y;
   const int32_t T = threadIdx.x;
@@ -874,6 +904,15 @@ __global__ __launch_bounds__(UT) void build_union_kernel(UnionArgs a) {
   if (!position && !group) part -= static_cast<int32_t>(a.Hkv) * a.entry_parts;
   const int32_t chunk = group ? part - kv * a.entry_parts : part;
   const bool masks_in_lds = g * k <= UMAXMASK;
+  // a list has at most the history's tokens and at most those of the pages its heads select
+  const int64_t c0 = static_cast<int64_t>(chunk) * a.chunk;
+  const int64_t most = static_cast<int64_t>(position ? Hq : g) * k * P;
+  if (position && c0 > 0 && (c0 >= L || c0 >= most)) {
+    const int64_t end = c0 + a.chunk < a.pos_cap ? c0 + a.chunk : a.pos_cap;
+    for (int64_t i = c0 + T; i < end; i += UT) a.positions[b * a.pos_cap + i] = -1;
+    return;
+  }
+  if (group && c0 > 0 && (c0 >= L || c0 >= most)) return;
   // page and row of a token offset: a shift where the page size is a power of two
   auto page_of = [&](uint32_t i) { return static_cast<int32_t>(a.pshift >= 0 ? i >> a.pshift : i / static_cast<uint32_t>(P)); };
 
@@ -900,8 +939,13 @@ __global__ __launch_bounds__(UT) void build_union_kernel(UnionArgs a) {
     }
   }
   __syncthreads();
-  if (T < 64) prefix_popcounts(ubits, uprefix, words);
-  else if (T < 128 && group) prefix_popcounts(gbits, gprefix, words);
+  if (!a.use_map) {
+    block_prefix_popcounts(ubits, uprefix, gbits, gprefix, words, reinterpret_cast<uint64_t*>(rank_page));
+  } else if (T < 64) {
+    prefix_popcounts(ubits, uprefix, words);
+  } else if (T < 128 && group) {
+    prefix_popcounts(gbits, gprefix, words);
+  }
   __syncthreads();
   auto rank_of = [&](const uint32_t* bits, const uint32_t* pre, int32_t p) -> int32_t {
     return static_cast<int32_t>(pre[p >> 5]) + __popc(bits[p >> 5] & ((1u << (p & 31)) - 1u));
@@ -919,9 +963,8 @@ __global__ __launch_bounds__(UT) void build_union_kernel(UnionArgs a) {
         for (int32_t w = T; w < words; w += UT) a.page_bits[b * a.pb_stride + w] = ubits[w];
     }
     // the chunk: `size` positions from c0, the first `held` of them union positions
-    const int64_t c0 = static_cast<int64_t>(chunk) * UCHUNK;
     int32_t* pos = a.positions + b * a.pos_cap + c0;
-    const int32_t size = a.pos_cap - c0 < UCHUNK ? static_cast<int32_t>(a.pos_cap - c0) : UCHUNK;
+    const int32_t size = a.pos_cap - c0 < a.chunk ? static_cast<int32_t>(a.pos_cap - c0) : a.chunk;
     const int32_t held = n <= c0 ? 0 : n - c0 < size ? static_cast<int32_t>(n - c0) : size;
     const int32_t i0 = static_cast<int32_t>(c0);  // used where held > 0: below n
     if (a.use_map) {
@@ -938,10 +981,10 @@ __global__ __launch_bounds__(UT) void build_union_kernel(UnionArgs a) {
         if (!((ubits[p >> 5] >> (p & 31)) & 1u)) continue;
         const int32_t base = rank_of(ubits, uprefix, p) * P;
         const int32_t plen = p == count - 1 ? tail_len : P;
-        for (int32_t off = 0; off < plen; ++off) {
-          const int64_t i = base + off - c0;
-          if (i >= 0 && i < held) pos[i] = p * P + off;
-        }
+        // the page's tokens in the chunk
+        const int64_t o0 = c0 - base > 0 ? c0 - base : 0;
+        const int64_t o1 = c0 + held - base < plen ? c0 + held - base : plen;
+        for (int64_t off = o0; off < o1; ++off) pos[base + off - c0] = static_cast<int32_t>(p * P + off);
       }
     }
     for (int32_t i = held + T; i < size; i += UT) pos[i] = -1;
@@ -968,9 +1011,9 @@ __global__ __launch_bounds__(UT) void build_union_kernel(UnionArgs a) {
       if (E > a.ecap) atomicOr(a.status, 2);
       if (a.estats) atomicAdd(a.estats, static_cast<unsigned long long>(held));
     }
-    if (static_cast<int64_t>(chunk) * UCHUNK >= held) return;
-    const uint32_t i0 = static_cast<uint32_t>(chunk) * UCHUNK;  // below held; the step past i1 may pass 31 bits
-    const uint32_t i1 = static_cast<uint32_t>(held) - i0 < UCHUNK ? static_cast<uint32_t>(held) : i0 + UCHUNK;
+    if (c0 >= held) return;
+    const uint32_t i0 = static_cast<uint32_t>(c0);  // below held; the step past i1 may pass 31 bits
+    const uint32_t i1 = held - c0 < a.chunk ? static_cast<uint32_t>(held) : i0 + a.chunk;
     if (masks_in_lds) {
       // head bits of each group page, indexed by the page's rank in the group
       for (int32_t i = T; i < g * k; i += UT) {
@@ -998,6 +1041,12 @@ __global__ __launch_bounds__(UT) void build_union_kernel(UnionArgs a) {
     for (int32_t p = T; p < count; p += UT) {
       if (!((gbits[p >> 5] >> (p & 31)) & 1u)) continue;
       const int32_t grank = rank_of(gbits, gprefix, p);
+      const int32_t gbase = grank * P;
+      const int32_t plen = p == count - 1 ? tail_len : P;
+      // the page's tokens in the chunk
+      const int64_t o0 = c0 - gbase > 0 ? c0 - gbase : 0;
+      const int64_t o1 = static_cast<int64_t>(i1) - gbase < plen ? static_cast<int64_t>(i1) - gbase : plen;
+      if (o0 >= o1) continue;
       uint32_t mask = 0u;
       if (masks_in_lds) {
         mask = gmask[grank];
@@ -1005,15 +1054,10 @@ __global__ __launch_bounds__(UT) void build_union_kernel(UnionArgs a) {
         for (int32_t hl = 0; hl < g; ++hl)
           if (head_has_page(pg + (kv * g + hl) * top, k, p)) mask |= 1u << hl;
       }
-      const int32_t gbase = grank * P;
       const int32_t ubase = rank_of(ubits, uprefix, p) * P;
-      const int32_t plen = p == count - 1 ? tail_len : P;
-      for (int32_t off = 0; off < plen; ++off) {
-        const uint32_t i = gbase + off;
-        if (i >= i0 && i < i1) {
-          ec[i] = ubase + off;
-          em[i] = mask;
-        }
+      for (int64_t off = o0; off < o1; ++off) {
+        ec[gbase + off] = static_cast<int32_t>(ubase + off);
+        em[gbase + off] = mask;
       }
     }
   }
@@ -1217,7 +1261,7 @@ static int build_union_chunk(const int32_t* pages, int64_t p_stride_b, int64_t t
   a.words = (max_count + 31) / 32;
   a.maxcount = max_count;
   a.use_map = max_count <= UMAPPAGES;
-  const size_t lds = static_cast<size_t>((4 * a.words + (a.use_map ? max_count : 0)) * 4);
+  const size_t lds = static_cast<size_t>((4 * a.words + (a.use_map ? max_count : 32)) * 4);
   static bool lds_attr = false;
   if (!lds_attr) {  // up to 4 * 768 + 24576 words of dynamic LDS
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(build_union_kernel),
@@ -1226,11 +1270,19 @@ static int build_union_chunk(const int32_t* pages, int64_t p_stride_b, int64_t t
     lds_attr = true;
   }
   a.pshift = (a.P & (a.P - 1)) == 0 ? __builtin_ctzll(static_cast<unsigned long long>(a.P)) : -1;
-  const int64_t pos_parts = ceil_div(pos_capacity, UCHUNK);
-  // a KV head has at most one entry per token
-  const int64_t entry_parts = ceil_div(std::min(entry_capacity, *std::max_element(lengths, lengths + batch)), UCHUNK);
-  a.part_heads = static_cast<int>(std::max<int64_t>(1, UCHUNK / width));
-  const int64_t parts = pos_parts + kv_heads * entry_parts + ceil_div(heads, a.part_heads);
+  // a list has at most one row per token of the longest history
+  const int64_t longest = *std::max_element(lengths, lengths + batch);
+  const int64_t most_pos = std::min(pos_capacity, longest), most_entries = std::min(entry_capacity, longest);
+  a.part_heads = static_cast<int>(std::max<int64_t>(1, UCHUNK / std::max<int64_t>(width, UT)));
+  const int64_t head_parts = ceil_div(heads, a.part_heads);
+  int64_t chunk = UCHUNK;
+  while (chunk < UCHUNK_MAX &&
+         batch * (ceil_div(most_pos, chunk) + kv_heads * ceil_div(most_entries, chunk) + head_parts) > UCUS)
+    chunk *= 2;
+  a.chunk = static_cast<int>(chunk);
+  const int64_t pos_parts = ceil_div(pos_capacity, chunk);  // what no history reaches is filled with -1
+  const int64_t entry_parts = ceil_div(most_entries, chunk);
+  const int64_t parts = pos_parts + kv_heads * entry_parts + head_parts;
   HS_CHECK_ARG(pos_parts <= INT32_MAX / 2 && parts <= INT32_MAX - UGRID, "union capacities too large");
   a.parts = static_cast<int>(parts);
   a.pos_parts = static_cast<int>(pos_parts);

@@ -511,11 +511,69 @@ def test_union_builder_matches_host_adapter(gpu, pages, P, kv, g, top, length):
         (900, 24, 1, 2, 200, 21590),  # several chunks of pages that are no power of two
         (6000, 3, 2, 3, 1500, None),  # a head's columns longer than a chunk
         (260, 16, 1, 16, 16, None),  # many heads of few columns per workgroup
+        (6000, 16, 40, 8, 100, None),  # more than a workgroup per CU: chunks of 8192
+        (3000, 16, 64, 8, 70, 47990),  # and of 16384
+        (30000, 16, 2, 2, 400, 479990),  # several chunks of a history beyond the LDS rank -> page map
     ],
 )
 def test_union_builder_chunk_edges(gpu, pages, P, kv, g, top, length):
     """Unions, entry lists and head columns at the edges of a workgroup's share."""
     test_union_builder_matches_host_adapter(gpu, pages, P, kv, g, top, length)
+
+
+@pytest.mark.parametrize("lengths,capacity", [([9599, 40, 4097], None), ([40, 9599], 20000), ([17], 20000)])
+def test_union_builder_of_ragged_histories(gpu, lengths, capacity):
+    """Chunks that only the longest history, or none, reaches: their positions are -1."""
+    from mini_hisparse_amd.selection import build_union
+
+    P, kv, g, top = 16, 2, 3, 300
+    rng = np.random.default_rng(len(lengths))
+    rows = np.full((len(lengths), kv * g, top), -1, np.int32)
+    for b, length in enumerate(lengths):
+        count = -(-length // P)
+        k = min(top, count)
+        for h in range(kv * g):
+            rows[b, h, :k] = np.append(np.sort(rng.permutation(count - 1)[: k - 1]), count - 1)
+    pages = torch.from_numpy(rows).to(gpu)
+    if capacity is None:
+        built = build_union(pages, lengths, P, kv, top)
+        results = [(t.positions, t.head_columns, t.union_count, t.entries) for t in built]
+    else:
+        results = _union_with_capacity(gpu, pages, lengths, P, kv, top, capacity)
+    for b, (positions, head_columns, union_count, entries) in enumerate(results):
+        k = min(top, -(-lengths[b] // P))
+        union, columns = oracle_union(pages_to_positions(rows[b, :, :k], lengths[b], P))
+        pos, hc = positions.cpu().numpy(), head_columns.cpu().numpy()
+        assert int(union_count) == len(union)
+        np.testing.assert_array_equal(pos[: len(union)], union)
+        assert (pos[len(union) :] == -1).all()
+        np.testing.assert_array_equal(hc[:, : columns.shape[1]], columns)
+        assert (hc[:, columns.shape[1] :] == -1).all()
+        for j, (cols, masks) in enumerate(group_entries(columns, kv)):
+            assert int(entries.counts[j]) == len(cols)
+            np.testing.assert_array_equal(entries.columns[j, : len(cols)].cpu().numpy(), cols)
+            np.testing.assert_array_equal(entries.masks[j, : len(cols)].cpu().numpy().astype(np.int64), masks)
+
+
+def _union_with_capacity(gpu, pages, lengths, P, kv, top, capacity):
+    """``hs_build_union`` into lists of ``capacity`` positions and entries."""
+    from mini_hisparse_amd import _lib
+    from mini_hisparse_amd.row_index import GroupEntries
+    from mini_hisparse_amd.selection import selection_width
+
+    B, heads = pages.shape[:2]
+    width = max(selection_width(n, P, top) for n in lengths)
+    new = lambda dtype, *shape: torch.full(shape, 77, dtype=dtype, device=gpu)  # noqa: E731
+    positions, columns = new(torch.int32, B, capacity), new(torch.int64, B, heads, width)
+    union_count, counts = new(torch.int32, B), new(torch.int32, B, kv)
+    ecol, emask, status = new(torch.int32, B, kv, capacity), new(torch.int32, B, kv, capacity), new(torch.int32, 1)
+    _lib.check(_lib.load().hs_build_union(
+        pages.data_ptr(), pages.stride(0), top, (ctypes.c_int64 * B)(*lengths), P, B, heads, kv, positions.data_ptr(),
+        capacity, columns.data_ptr(), width, union_count.data_ptr(), ecol.data_ptr(), emask.data_ptr(), capacity,
+        counts.data_ptr(), status.data_ptr(), None, 0, None, _lib.stream_handle(gpu)), "hs_build_union")
+    assert status.item() == 77  # nothing overflowed
+    return [(positions[b], columns[b], union_count[b], GroupEntries(ecol[b], emask[b], counts[b], capacity))
+            for b in range(B)]
 
 
 @pytest.mark.parametrize("top,P,length", [(2**32 + 1, 16, 40), (3, 2**33, 5), (2**32, 2**32 + 1, 7)])
