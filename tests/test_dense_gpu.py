@@ -372,10 +372,10 @@ def test_projection_rows_across_tile_edges(gpu, rows, n, k):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n", [16, 32800, 262144, 262176])
+@pytest.mark.parametrize("n", [16, 8192, 32768, 32800, 262144, 262176])
 def test_argmax_key_counts(gpu, n):
-    """The argmax's last step at one key per token, several, a full round of its loads and
-    one more; the largest logit planted in the last rows."""
+    """The argmax's last step at one key per token, several, the most that take 256 threads and
+    the least that take more, a full round of its loads and one more; the largest logit planted in the last rows."""
     from mini_hisparse_amd.dense import linear_argmax_tiled, tile_weight
 
     w = torch.randn(n, 32, generator=torch.Generator(device=gpu).manual_seed(n), device=gpu).to(torch.bfloat16)
