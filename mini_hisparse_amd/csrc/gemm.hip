@@ -30,6 +30,7 @@
 namespace hs {
 
 constexpr int GM_T = 256;  // threads per workgroup of gemm_finalize_kernel
+constexpr int GM_SLICES = 3;  // most K slices of a plan
 
 template <int DT>
 __device__ __forceinline__ f32x4 gemm_mfma(u32x4 a, u32x4 b, f32x4 c) {
@@ -235,7 +236,6 @@ __global__ __launch_bounds__(64 * NW) void skinny_gemm_kernel(GemmArgs a) {
     if (threadIdx.x == 0) s_last = arrive_last(a.counters + blockIdx.x, c0, a.epoch, a.splits) ? 1 : 0;
     __syncthreads();
     if (!s_last) return;
-    constexpr int MS = 8;  // slices whose words are loaded together
     const int64_t sstride = a.M * a.N;
     for (int idx = threadIdx.x; idx < GM_ROWS * 16; idx += GM_T) {
       const int r = idx >> 4, m = idx & 15;
@@ -243,19 +243,16 @@ __global__ __launch_bounds__(64 * NW) void skinny_gemm_kernel(GemmArgs a) {
       if (m >= a.M || dropped(n)) continue;
       const unsigned long long* w0 = a.words + m * a.N + n;
       float v = 0.f;
-      for (int64_t s0 = 0; s0 < a.splits; s0 += MS) {
-        unsigned long long w[MS];
+      unsigned long long w[GM_SLICES];  // every slice's word, loaded together
 #pragma unroll
-        for (int u = 0; u < MS; ++u) {
-          const int64_t sl = s0 + u < a.splits ? s0 + u : s0;  // in bounds; not added
-          w[u] = __hip_atomic_load(w0 + sl * sstride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+      for (int u = 0; u < GM_SLICES; ++u)
+        if (u < a.splits)
+          w[u] = __hip_atomic_load(w0 + u * sstride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
-        for (int u = 0; u < MS; ++u) {
-          if (s0 + u >= a.splits) break;
-          if (static_cast<uint32_t>(w[u] >> 32) != tag) w[u] = partial_reread(w0 + (s0 + u) * sstride, tag);
-          v += partial_value(w[u]);
-        }
+      for (int u = 0; u < GM_SLICES; ++u) {
+        if (u >= a.splits) break;
+        if (static_cast<uint32_t>(w[u] >> 32) != tag) w[u] = partial_reread(w0 + u * sstride, tag);
+        v += partial_value(w[u]);
       }
       const float b = a.bias != nullptr ? load_elem<DT>(a.bias, n) : 0.f;
       store_elem<DT>(a.out, m * a.out_stride + n, v + b);
@@ -363,10 +360,10 @@ static GemmPlan plan_gemm(int64_t N, int64_t K, bool one_slice = false) {
   constexpr uint64_t CUS = 256, X_SHARE = 8, MERGE = 48, LONG_SLICE = 256;
   const uint64_t steps = static_cast<uint64_t>(K) / 32;
   const uint64_t n[2] = {(static_cast<uint64_t>(N) + 15) / 16, (static_cast<uint64_t>(N) + 31) / 32};
-  const uint64_t slices[3] = {steps, (steps + 1) / 2, (steps + 2) / 3};
+  const uint64_t slices[GM_SLICES] = {steps, (steps + 1) / 2, (steps + 2) / 3};
   GemmPlan p{};
   uint64_t best = UINT64_MAX;
-  for (uint64_t s = 1; s <= (one_slice ? 1u : 3u); ++s) {
+  for (uint64_t s = 1; s <= (one_slice ? 1 : GM_SLICES); ++s) {
     const uint64_t slice = slices[s - 1];
     if (slice * (s - 1) >= steps) break;  // a slice would be empty
     for (uint64_t tiles = 2; tiles >= 1; --tiles) {
