@@ -30,7 +30,7 @@
 namespace hs {
 
 constexpr int GM_T = 256;  // threads per workgroup of gemm_finalize_kernel
-constexpr int GM_SLICES = 3;  // most K slices of a plan
+constexpr int GM_SLICES = 8;  // most K slices of a plan
 
 template <int DT>
 __device__ __forceinline__ f32x4 gemm_mfma(u32x4 a, u32x4 b, f32x4 c) {
@@ -340,37 +340,48 @@ static int64_t gemm_ceil(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Waves of a workgroup: 8 where a wave of 4 would read its k-steps in more than one round
 // (each round is a memory round trip, and a CU with one workgroup has only its own waves'
-// loads in flight), unless there are so many rows that every CU holds several workgroups.
+// loads in flight), unless there are so many rows that every CU holds several workgroups
+// (then only for steps that fill the 8 waves' first round too).
 // 8 rows, us with 4 and with 8 waves: 3584 x 3584 9.8 and 8.5, 896 x 4864 10.5 and 8.3,
-// 3584 x 18944 39.4 and 30.0; 1152 x 896 (7 steps a wave of 4) 3.60 and 3.65.  The same for
-// a projection in one K slice and its fused forms, so their sums agree.
-static int gemm_waves(int64_t N, int64_t slice_steps) { return slice_steps > 32 && N <= 16384 ? 8 : 4; }
+// 3584 x 18944 39.4 and 30.0; 1152 x 896 (7 steps a wave of 4) 3.60 and 3.65; one tile of
+// 12288 x 1536 9.3 and 10.9.  The same for a projection in one K slice and its fused forms,
+// so their sums agree.
+static int gemm_waves(int64_t N, int64_t slice_steps) {
+  return slice_steps > 32 && (N <= 8192 || (slice_steps > 64 && N <= 16384)) ? 8 : 4;
+}
 
 // Row tiles of 16 per workgroup and K slices.  The weight's stream bounds the launch, a CU
 // reads about 23 bytes per ns, and the launch ends with the CU that reads most: the cost of
 // a plan is the rounds of its workgroups over the 256 CUs times a workgroup's tile-steps
 // (1 KB each), an eighth more with one tile, which reads x twice as often per weight byte.
-// Merging K slices costs about 48 tile-steps (2 us), and pays only within one round or for
-// long slices.  Measured, 8 rows, us before (at least 512 workgroups of 4 waves) and with
-// these plans: 3584 x 18944 34.2 and 29.6 (two tiles in two slices instead of one in three),
-// 7168 x 5120 21.6 and 15.7, 5120 x 27648 64.9 and 53.3 (two tiles in three slices),
-// 896 x 4864 9.6 and 7.5 (three slices), 3584 x 3584 9.9 and 8.1.
+// A second tile costs about 24 tile-steps (1 us of loads, LDS sums and stores) whatever K is.
+// Merging K slices costs about 48 (2 us), and pays only within one round or for long slices;
+// more than three only while each keeps 96 k-steps (few rows of a long K).
+// Measured, 8 rows, us with at least 512 workgroups of 4 waves (one tile up to 16384 rows) and
+// with these plans: 3584 x 18944 34.2 and 28.5 (two tiles in two slices instead of one in
+// three), 7168 x 5120 21.6 and 15.7, 5120 x 27648 64.9 and 53.3 (two tiles in three slices),
+// 896 x 4864 9.6 and 7.5 (three slices); without the second tile's share 8192 x 512 takes two
+// tiles, 4.4 and 5.1, with it one, 4.4; with at most three slices 16 x 27648 12.0 instead of
+// 8.1, with eight 7.5.
 static GemmPlan plan_gemm(int64_t N, int64_t K, bool one_slice = false) {
   // unsigned, with constant divisors: every projection call plans, on the host's time
-  constexpr uint64_t CUS = 256, X_SHARE = 8, MERGE = 48, LONG_SLICE = 256;
+  constexpr uint64_t CUS = 256, X_SHARE = 8, TILE2 = 24, MERGE = 48, LONG_SLICE = 256, MORE_SLICES = 96;
   const uint64_t steps = static_cast<uint64_t>(K) / 32;
   const uint64_t n[2] = {(static_cast<uint64_t>(N) + 15) / 16, (static_cast<uint64_t>(N) + 31) / 32};
-  const uint64_t slices[GM_SLICES] = {steps, (steps + 1) / 2, (steps + 2) / 3};
+  const uint64_t slices[GM_SLICES] = {steps, (steps + 1) / 2, (steps + 2) / 3, (steps + 3) / 4, (steps + 4) / 5,
+                                      (steps + 5) / 6, (steps + 6) / 7, (steps + 7) / 8};
+  // Many rows of a short K: 20480 x 512 in one tile 7.7 us, in two 6.9
+  const bool two_tiles = N > 16384 && steps <= 16;
   GemmPlan p{};
   uint64_t best = UINT64_MAX;
   for (uint64_t s = 1; s <= (one_slice ? 1 : GM_SLICES); ++s) {
     const uint64_t slice = slices[s - 1];
-    if (slice * (s - 1) >= steps) break;  // a slice would be empty
-    for (uint64_t tiles = 2; tiles >= 1; --tiles) {
+    if (slice * (s - 1) >= steps || (s > 3 && slice < MORE_SLICES)) break;  // one would be empty, or too short
+    for (uint64_t tiles = 2; tiles >= (two_tiles ? 2u : 1u); --tiles) {
       const uint64_t blocks = n[tiles - 1];
       if (s > 1 && blocks * s > CUS && slice < LONG_SLICE) continue;
       const uint64_t stream = (blocks * s + CUS - 1) / CUS * slice * tiles;
-      const uint64_t cost = stream + (tiles == 1 ? stream / X_SHARE : 0) + (s > 1 ? MERGE : 0);
+      const uint64_t cost = stream + (tiles == 1 ? stream / X_SHARE : TILE2) + (s > 1 ? MERGE : 0);
       if (cost >= best) continue;
       best = cost;
       p.tiles = static_cast<int>(tiles);
@@ -385,10 +396,14 @@ static GemmPlan plan_gemm(int64_t N, int64_t K, bool one_slice = false) {
   // 12.2 and 10.3 (14.2 and 12.2), 5120 x 5120 15.9 and 13.6 (19.2 and 16.9), 6144 x 4096 13.2
   // and 12.6 (15.9 and 14.5).  Fewer rows than a tile's, or two rounds, do not pay: the second
   // tile's loads cost more than the bytes they leave out (3584 x 3584 in one tile 8.0, in
-  // 14 rows of two 9.7; 9216 x 4096 19.0 and 20.7).  Longer K stays in slices.
+  // 14 rows of two 9.7; 9216 x 4096 19.0 and 20.7), so they are charged 36 here, which leaves
+  // K up to 1024 to one tile (5120 x 512 4.2, even rows 4.9; 4608 x 1024 5.2 and 5.5).  Longer
+  // K stays in slices: 5120 x 27648 in three 50.1, in 20 rows 53.3 (but 4608 x 18944, here two
+  // whole tiles and one slice, 41.0 and in 18 rows 36.1).
+  constexpr uint64_t EVEN = 36;
   uint64_t rows = 2 * ((static_cast<uint64_t>(N) + 2 * CUS - 1) / (2 * CUS));
   if (rows == 22) rows = 24;  // starts at multiples of 2: 22 rows could touch a third tile
-  if (!one_slice && rows > 16 && rows <= 24 && steps <= 2 * LONG_SLICE && steps * rows / 16 < best) {
+  if (!one_slice && rows > 16 && rows <= 24 && steps <= 2 * LONG_SLICE && steps * rows / 16 + EVEN < best) {
     p.tiles = 2;
     p.rows = static_cast<int64_t>(rows);
     p.blocks = gemm_ceil(N, p.rows);
