@@ -394,20 +394,26 @@ __device__ __forceinline__ uint32_t score_key(float s) {
 // pages written ascending; the tail page and the sink are always taken.
 //
 // A thread holds its keys in registers (page j * TT + thread), so the scores are read
-// once.  What bounds the launch is its chain of block-wide steps, so there are few:
-// the least and largest key give a range that one histogram of 2048 equal bins covers
-// (a head's scores crowd into a few powers of two, where fixed top digits of the key put
-// most pages into a handful of bins and a lane's LDS atomics behind each other's), the bin
-// holding the last taken key is found by one scan from the top, and usually holds few
-// keys: they are ranked among themselves.  A bin of more than TOPK_FEW keys is cut into
-// 2048 again; equal keys are ranked by page.  Every wave's taken pages are a ballot, and
+// once.  What bounds the launch is its chain of block-wide steps, so there are few: a lower
+// bound of the last taken key and the largest key give a range that one histogram of 2048
+// equal bins covers (a head's scores crowd into a few powers of two, where fixed top digits
+// of the key put most pages into a handful of bins and a lane's LDS atomics behind each
+// other's), the bin holding the last taken key is found by one scan from the top, and usually
+// holds few keys: they are ranked among themselves.  A bin of more than FEW keys is cut
+// into 2048 again; equal keys are ranked by page.  Every wave's taken pages are a ballot, and
 // the ballots of (j, wave) follow the pages' order, so one scan of their counts places
 // each page.
-// Measured (kernel trace, top 64 of 8192 pages, 28 heads x 16 requests): 11.6 us, against
-// 25.8 us for the radix select of four 8-bit digits over keys in LDS; 2048 pages, 14 heads
-// x 4 requests: 5.7 against 10.9 us.
+// The bound: of `need` or more groups of keys, each holds a key at or above the least of the
+// groups' largest, so that many keys lie there and the last taken one does.  From the least
+// key instead, scores of both signs spread the bins over all powers of two down to zero.
+// us of the scorer and the top-k (28 heads, D = 128, top 64), radix select of four 8-bit digits
+// over keys in LDS / this from the least key, 64 keys ranked by a thread each / now:
+//   4 requests of 300 pages    one sign 14.4 / 10.6 / 10.8    both signs 14.4 / 15.3 / 12.2
+//   4 requests of 2048 pages            16.8 / 11.7 / 11.7               16.9 / 17.9 / 11.6
+//   4 requests of 8192 pages            32.6 / 22.0 / 21.5               33.1 / 28.6 / 21.3
+//   16 requests of 12000 pages, all scores equal 99.8 / 106.7 / 84.5
 constexpr int TOPK_BINS = 2048;
-constexpr int TOPK_FEW = 64;
+constexpr int TOPK_GROUP = 8;  // threads
 
 // cnt[0 .. N) -> its exclusive prefix sum, by the first wave.
 template <int N>
@@ -433,10 +439,13 @@ __device__ __forceinline__ void prefix_counts(int32_t* cnt) {
 template <int TT, int KPT>
 __global__ __launch_bounds__(TT, 4) void quest_topk_kernel(QuestArgs a) {  // at most 128 VGPRs
   constexpr int NW = TT / 64, PB = TOPK_BINS / TT;
+  // Keys ranked among themselves: more where few keys per thread leave no closer bound (300 pages,
+  // both signs, as above with 64: 15.6 us).
+  constexpr int FEW = KPT <= 2 ? 128 : 64;
   static_assert(KPT * TT <= 32 * TOPK_BINS, "the histogram also holds a bitmap of the pages");
   __shared__ uint32_t hist[TOPK_BINS];
   __shared__ uint32_t red[2 * NW];
-  __shared__ uint32_t few_key[TOPK_FEW], few_page[TOPK_FEW];
+  __shared__ uint32_t few_key[FEW], few_page[FEW];
   __shared__ int32_t cnt[KPT * NW];
   __shared__ uint32_t s_bin, s_above, s_held, s_few;
   const int64_t h = blockIdx.x, b = blockIdx.y;
@@ -470,11 +479,24 @@ __global__ __launch_bounds__(TT, 4) void quest_topk_kernel(QuestArgs a) {  // at
       hi = key[j] > hi ? key[j] : hi;
     }
   }
+  // still to take among the live keys
+  uint32_t need = static_cast<uint32_t>(a.top) - (sink ? 2u : 1u);
+  // The least of the largest keys of `need` or more groups of keys is a lower bound of the last
+  // taken key, and a far closer one than the least key: groups of TOPK_GROUP threads, or single
+  // threads (a group without a live key makes the bound 0).
+  const bool by_group = need <= TT / TOPK_GROUP && count >= TT;
+  const bool by_thread = need <= TT && count >= 2 * TT;
+  if (by_group || by_thread) lo = hi;
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    const uint32_t l = __shfl_xor(lo, off, 64), u = __shfl_xor(hi, off, 64);
-    lo = l < lo ? l : lo;
+  for (int off = 1; off <= 32; off <<= 1) {
+    const uint32_t u = __shfl_xor(hi, off, 64);
     hi = u > hi ? u : hi;
+    if (by_group && off < TOPK_GROUP) {
+      lo = hi;
+    } else {
+      const uint32_t l = __shfl_xor(lo, off, 64);
+      lo = l < lo ? l : lo;
+    }
   }
   if (lane == 0) {
     red[wave] = lo;
@@ -486,10 +508,29 @@ __global__ __launch_bounds__(TT, 4) void quest_topk_kernel(QuestArgs a) {  // at
     lo = red[w] < lo ? red[w] : lo;
     hi = red[NW + w] > hi ? red[NW + w] : hi;
   }
-  // still to take among the live keys, all of which lie in [lo, hi]
-  uint32_t need = static_cast<uint32_t>(a.top) - (sink ? 2u : 1u);
+  // the keys that may still be taken lie in [lo, hi]
+#pragma unroll
+  for (int j = 0; j < KPT; ++j)
+    if (key[j] < lo) live &= ~(1u << j);
   uint32_t span = hi > lo ? hi - lo : 0u;
   while (need > 0) {  // the same for the whole workgroup
+    if (span == 0u) {  // equal keys: the lowest pages
+#pragma unroll 1
+      for (int j = 0; j < KPT; ++j) {
+        const uint64_t m = __ballot((live >> j) & 1u);
+        if (lane == 0) cnt[j * NW + wave] = __popcll(m);
+      }
+      __syncthreads();
+      prefix_counts<KPT * NW>(cnt);
+      __syncthreads();
+#pragma unroll 1
+      for (int j = 0; j < KPT; ++j) {
+        const uint64_t m = __ballot((live >> j) & 1u);
+        if (((live >> j) & 1u) && static_cast<uint32_t>(cnt[j * NW + wave] + lanes_below(m)) < need) taken |= 1u << j;
+      }
+      __syncthreads();  // cnt is written again below
+      break;
+    }
     const int bits = 32 - __clz(static_cast<int>(span));  // __clz(0) == 32
     const int shift = bits > 11 ? bits - 11 : 0;
 #pragma unroll
@@ -523,6 +564,7 @@ __global__ __launch_bounds__(TT, 4) void quest_topk_kernel(QuestArgs a) {  // at
     __syncthreads();
     const uint32_t bin = s_bin, held = s_held;
     need -= s_above;
+    asm volatile("" : "+v"(lo));  // the keys' bins are taken again: kept, 18 keys a thread spill
 #pragma unroll
     for (int j = 0; j < KPT; ++j) {
       const uint32_t k = (key[j] - lo) >> shift;
@@ -530,7 +572,7 @@ __global__ __launch_bounds__(TT, 4) void quest_topk_kernel(QuestArgs a) {  // at
       if (k != bin) live &= ~(1u << j);
     }
     if (held == need) break;
-    if (held <= TOPK_FEW) {  // rank the bin's keys among themselves
+    if (held <= FEW) {  // rank the bin's keys among themselves
 #pragma unroll
       for (int j = 0; j < KPT; ++j)
         if ((live >> j) & 1u) {
@@ -539,31 +581,30 @@ __global__ __launch_bounds__(TT, 4) void quest_topk_kernel(QuestArgs a) {  // at
           few_page[i] = static_cast<uint32_t>(j * TT + T);
         }
       __syncthreads();
-      if (static_cast<uint32_t>(T) < held) {
-        const uint32_t k = few_key[T], p = few_page[T];
+      // every wave holds them all, and ranks every NW-th of them by ballots
+      constexpr int FJ = FEW / 64;
+      uint32_t fk[FJ], fp[FJ];
+#pragma unroll
+      for (int i = 0; i < FJ; ++i) {
+        fk[i] = few_key[i * 64 + lane];
+        fp[i] = few_page[i * 64 + lane];
+      }
+      const int32_t mine = wave + NW * lane < FEW ? wave + NW * lane : 0;
+      const uint32_t mk = few_key[mine], mp = few_page[mine];
+      for (int32_t c = 0; wave + NW * c < static_cast<int32_t>(held); ++c) {
+        const uint32_t k = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(mk), c));
+        const uint32_t p = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(mp), c));
         uint32_t rank = 0;
-        for (uint32_t i = 0; i < held; ++i) rank += few_key[i] > k || (few_key[i] == k && few_page[i] < p);
-        if (rank < need) atomicOr(&hist[p >> 5], 1u << (p & 31));  // cleared above: a bitmap of the pages
+#pragma unroll
+        for (int i = 0; i < FJ; ++i) {
+          const bool before = fk[i] > k || (fk[i] == k && fp[i] < p);
+          rank += static_cast<uint32_t>(__popcll(__ballot(i * 64u + lane < held && before)));
+        }
+        if (lane == 0 && rank < need) atomicOr(&hist[p >> 5], 1u << (p & 31));  // cleared above: a bitmap of the pages
       }
       __syncthreads();
 #pragma unroll
       for (int j = 0; j < KPT; ++j) taken |= ((hist[(j * TT + T) >> 5] >> (T & 31)) & 1u) << j;
-      break;
-    }
-    if (shift == 0) {  // equal keys: the lowest pages
-      uint64_t m[KPT];
-#pragma unroll
-      for (int j = 0; j < KPT; ++j) {
-        m[j] = __ballot((live >> j) & 1u);
-        if (lane == 0) cnt[j * NW + wave] = __popcll(m[j]);
-      }
-      __syncthreads();
-      prefix_counts<KPT * NW>(cnt);
-      __syncthreads();
-#pragma unroll
-      for (int j = 0; j < KPT; ++j)
-        if (((live >> j) & 1u) && static_cast<uint32_t>(cnt[j * NW + wave] + lanes_below(m[j])) < need) taken |= 1u << j;
-      __syncthreads();  // cnt is written again below
       break;
     }
     lo += bin << shift;

@@ -440,7 +440,10 @@ def _score_pages(kind, pages, gen):
 @pytest.mark.parametrize("kind", ["normal", "spread", "crowd", "inf"])
 @pytest.mark.parametrize("pages,top", [(2, 1), (66, 65), (512, 8), (513, 8), (1024, 64), (1025, 64), (2048, 3),
                                        (2049, 64), (4096, 200), (4097, 64), (8192, 64), (8193, 64), (9216, 64),
-                                       (9217, 64), (16384, 5000), (16385, 64)])
+                                       (9217, 64), (16384, 5000), (16385, 64),
+                                       # as many pages to take as groups of threads, as threads, and one more
+                                       (512, 66), (1100, 66), (1100, 67), (1100, 514), (1100, 515), (10000, 130),
+                                       (10000, 131), (10000, 1026), (10000, 1027)])
 def test_quest_topk_page_counts_and_score_spreads(gpu, kind, pages, top):
     """Every register variant of the top-k at its first and last page count, over scores that
     need one cut of their range or several, or fill a bin."""
@@ -454,6 +457,35 @@ def test_quest_topk_page_counts_and_score_spreads(gpu, kind, pages, top):
     expected = oracle.quest_pages(q, bounds, bounds, pages * 16, 16, top)
     sel = quest_selection(q.to(gpu), bounds.to(gpu), bounds.to(gpu), pages * 16, 16, top)
     np.testing.assert_array_equal(sel.device_pages[:, : expected.shape[1]].cpu().numpy(), expected)
+
+
+@pytest.mark.parametrize("pages,alike", [(700, 2), (700, 64), (700, 65), (700, 128), (700, 129), (1100, 64), (1100, 65), (9300, 64),
+                                         (9300, 65), (40, 38), (700, 698), (1200, 1198)])
+def test_quest_topk_cut_inside_a_crowd(gpu, pages, alike):
+    """The last taken page is one of `alike` pages of eight close scores between one score far above
+    and others far below: ranked among themselves up to 128 or (above 1024 pages) 64 of them, cut
+    again beyond; where all but the forced pages are alike, of one score."""
+    from mini_hisparse_amd.selection import quest_selection
+
+    gen = torch.Generator().manual_seed(pages + alike)
+    x = -(10.0 ** (-3 * torch.rand(pages, generator=gen)))
+    crowd = 1 + torch.randperm(pages - 2, generator=gen)[:alike]  # neither the sink nor the tail
+    if alike < pages - 2:
+        x[crowd] = 1 + torch.randint(0, 8, (alike,), generator=gen) / 128
+        rest = torch.ones(pages, dtype=torch.bool)
+        rest[crowd] = rest[0] = rest[-1] = False
+        x[int(rest.nonzero()[0])] = 1e30
+        x[int(rest.nonzero()[-1])] = -1e30
+    else:
+        x[crowd] = 1.0
+    bounds = torch.zeros(pages, 2, 8, dtype=torch.bfloat16)
+    bounds[:, :, 0] = x[:, None].to(torch.bfloat16)
+    q = torch.zeros(4, 8, dtype=torch.bfloat16)
+    q[:, 0] = torch.tensor([1.0, 0.5, 1.0, 2.0])
+    for top in sorted({4, alike // 2 + 3, min(alike + 2, pages - 1)}):
+        expected = oracle.quest_pages(q, bounds, bounds, pages * 16, 16, top)
+        sel = quest_selection(q.to(gpu), bounds.to(gpu), bounds.to(gpu), pages * 16, 16, top)
+        np.testing.assert_array_equal(sel.device_pages[:, : expected.shape[1]].cpu().numpy(), expected)
 
 
 def test_quest_reference_known_answer(gpu):
