@@ -260,22 +260,27 @@ __global__ __launch_bounds__(QT) void quest_score_tile_kernel(QuestArgs a) {
 // The launch is bound by the bounds' HBM stream: what it needs is loads in flight while
 // other waves score.  A 256-byte row (D = 128) is staged in PARTS = 2 halves of 128 bytes,
 // so a workgroup holds 36.9 KB of LDS, four share a CU instead of two, and the second
-// half's loads are in flight while the first is scored.  The bounds are read once per
-// launch, so their loads are non-temporal.  16 requests of 8192 pages, 28 heads, 4 KV heads
-// (268 MB): 66.2 us with whole rows, 55.4 us in halves (page tiles the fastest grid
-// dimension: 54.0), 50.7 us non-temporal = 5.3 TB/s; 8, 4 and 2 requests: 32.0, 19.7 and
-// 13.0 us in halves, 29.4, 18.6 and 12.3 us non-temporal.  Same arithmetic and order as
-// quest_score_kernel.
+// half's loads are in flight while the first is scored.  16 requests of 8192 pages, 28 heads,
+// 4 KV heads (268 MB): 66.2 us with whole rows, 55.4 us in halves (page tiles the fastest grid
+// dimension: 54.0).
+// NT, non-temporal loads, where one workgroup is the only reader of its lines (rows of whole
+// lines, D = 64 or 128, and one head chunk per KV head) and the bounds are too many to be in an
+// L2 still: the same 50.7 us = 5.3 TB/s; 8, 4 and 2 requests: 32.0, 19.7 and 13.0 us without,
+// 29.4, 18.6 and 12.3 us with.  Elsewhere they cost (us with the top-k of one page, 16 requests of
+// 8192 pages, without and with): 32 heads on one KV head, four chunks, 63.8 and 70.4; 8 KV heads
+// of D = 32, two rows to a line, 48.8 and 54.7; a megabyte (1 request of 2048 pages, 2 KV heads of
+// D = 64) 7.4 and 8.3.  Same arithmetic and order as quest_score_kernel.
 constexpr int QP_PAGES = 128;                // pages per workgroup: two per lane
 constexpr int QP_T = 64 * QHEADS;            // one wave per query head of the chunk
 constexpr int QP_UNITS = 4;                  // 16-byte units per thread, bound and staging round
+constexpr int64_t QP_NT_BYTES = 2 << 20;     // least bounds of a launch that are read non-temporally
 constexpr int64_t QP_MAX_ROW_BYTES = 256;    // D <= 128: one staging round per part
 
 __host__ __device__ constexpr int64_t qp_lds_bytes(int64_t row_bytes, int parts) {
   return 2 * QP_PAGES * (row_bytes / parts + 16);
 }
 
-template <bool QF32, int DK, int PARTS>
+template <bool QF32, int DK, int PARTS, bool NT>
 __global__ __launch_bounds__(QP_T, 4 * PARTS) void quest_score_perm_kernel(QuestArgs a) {
 #pragma clang fp contract(off)
   extern __shared__ __attribute__((aligned(16))) unsigned char qp_smem[];
@@ -308,8 +313,10 @@ __global__ __launch_bounds__(QP_T, 4 * PARTS) void quest_score_perm_kernel(Quest
       if (u >= units) u = 0;
       const uint32_t r = u / upr, c = u - r * upr;
       const uint64_t off = static_cast<uint64_t>(r) * gstride + (part * upr + c) * 16u;
-      Ls[k] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(lo_t + off));
-      Us[k] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(hi_t + off));
+      const u32x4* lo_at = reinterpret_cast<const u32x4*>(lo_t + off);
+      const u32x4* hi_at = reinterpret_cast<const u32x4*>(hi_t + off);
+      Ls[k] = NT ? __builtin_nontemporal_load(lo_at) : *lo_at;
+      Us[k] = NT ? __builtin_nontemporal_load(hi_at) : *hi_at;
     }
   };
   auto stage = [&]() {
@@ -1183,15 +1190,19 @@ static int quest_topk_chunk(const void* query, int64_t q_stride_b, int64_t q_str
                 static_cast<unsigned>(batch));
       const size_t lds = static_cast<size_t>(qp_lds_bytes(row_bytes, head_dim == 128 ? 2 : 1));
       const bool f32q = query_dtype == HS_DTYPE_F32;
+      int64_t bound_rows = 0;
+      for (int64_t i = 0; i < batch; ++i) bound_rows += page_counts[i];
+      const bool nt = hchunks == 1 && bound_rows * kv_heads * row_bytes * 2 >= QP_NT_BYTES;
+      auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(QP_T), lds, stream, a); };
       if (head_dim == 128) {
-        if (f32q) hipLaunchKernelGGL((quest_score_perm_kernel<true, 128, 2>), grid, dim3(QP_T), lds, stream, a);
-        else hipLaunchKernelGGL((quest_score_perm_kernel<false, 128, 2>), grid, dim3(QP_T), lds, stream, a);
+        if (f32q) nt ? launch(quest_score_perm_kernel<true, 128, 2, true>) : launch(quest_score_perm_kernel<true, 128, 2, false>);
+        else nt ? launch(quest_score_perm_kernel<false, 128, 2, true>) : launch(quest_score_perm_kernel<false, 128, 2, false>);
       } else if (head_dim == 64) {
-        if (f32q) hipLaunchKernelGGL((quest_score_perm_kernel<true, 64, 1>), grid, dim3(QP_T), lds, stream, a);
-        else hipLaunchKernelGGL((quest_score_perm_kernel<false, 64, 1>), grid, dim3(QP_T), lds, stream, a);
+        if (f32q) nt ? launch(quest_score_perm_kernel<true, 64, 1, true>) : launch(quest_score_perm_kernel<true, 64, 1, false>);
+        else nt ? launch(quest_score_perm_kernel<false, 64, 1, true>) : launch(quest_score_perm_kernel<false, 64, 1, false>);
       } else {
-        if (f32q) hipLaunchKernelGGL((quest_score_perm_kernel<true, 0, 1>), grid, dim3(QP_T), lds, stream, a);
-        else hipLaunchKernelGGL((quest_score_perm_kernel<false, 0, 1>), grid, dim3(QP_T), lds, stream, a);
+        if (f32q) launch(quest_score_perm_kernel<true, 0, 1, false>);
+        else launch(quest_score_perm_kernel<false, 0, 1, false>);
       }
       HS_CHECK_LAUNCH("quest scorer");
     } else if (head_dim % epv == 0 && aligned && row_bytes <= QS_MAX_ROW_BYTES) {

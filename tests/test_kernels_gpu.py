@@ -372,6 +372,11 @@ def test_quest_pages_match_oracle(gpu, dtype, pages, P, kv, g, D, top, sink, len
         (torch.bfloat16, [2048, 300, 77], 2, 7, 64),  # 0.5B geometry
         (torch.float32, [300], 1, 12, 64),  # two head chunks per KV head
         (torch.bfloat16, [130], 3, 5, 40),  # D = 40: five 16-byte units per row
+        (torch.bfloat16, [300, 77], 1, 12, 128),  # two head chunks of rows staged in halves
+        (torch.float32, [129], 1, 16, 128),
+        (torch.bfloat16, [511, 512], 4, 7, 128),  # a page less than the least bounds read non-temporally
+        (torch.bfloat16, [512, 512], 4, 7, 128),  # as many
+        (torch.float32, [4000, 97], 2, 7, 64),
     ],
 )
 def test_quest_scores_bit_exact(gpu, q_dtype, counts, kv, g, D):
