@@ -293,13 +293,11 @@ __global__ __launch_bounds__(GM_T) void gemm_finalize_kernel(const float* part, 
 
 // One workgroup per token: the largest of its `blocks` keys, as the vocabulary index.
 // Bound by the round trips of its loads: FIN_KEYS keys per thread are loaded together
-// (4752 keys a token: 4.8 us, 9.2 us with 256 threads of one load at a time).  Up to
-// FIN_FEW keys take 256 threads, whose fewer waves start and meet sooner (16 keys, with the
-// product of 256 x 128: 5.1 us with 1024 threads, 4.8 with 256).
-constexpr int FIN_KEYS = 8;
-constexpr int64_t FIN_FEW = 1024;
-
-template <int FIN_T>
+// (4752 keys a token: 4.8 us, 9.2 us with 256 threads of one load at a time).  Up to 1024
+// keys take 256 threads, whose fewer waves start and meet sooner, and up to 256 one load each
+// (16 keys, with the product of 256 x 128: 5.1 us with 1024 threads, 4.8 with 256 of 8 loads,
+// 4.7 with 256 of one).
+template <int FIN_T, int FIN_KEYS>
 __global__ __launch_bounds__(FIN_T) void argmax_finalize_kernel(const unsigned long long* keys, int64_t blocks,
                                                                 int64_t* tokens) {
   __shared__ unsigned long long wave_best[FIN_T / 64];
@@ -615,8 +613,12 @@ extern "C" int hs_skinny_gemm_argmax_tiled(const void* x, int64_t x_stride, cons
   else launch_gemm<HS_DTYPE_F16, true, true>(p, grid, a, stream);
   HS_CHECK_LAUNCH("skinny GEMM argmax");
   const dim3 fin(static_cast<unsigned>(rows));
-  if (p.blocks <= FIN_FEW) hipLaunchKernelGGL(argmax_finalize_kernel<256>, fin, dim3(256), 0, stream, a.keys, p.blocks, tokens);
-  else hipLaunchKernelGGL(argmax_finalize_kernel<1024>, fin, dim3(1024), 0, stream, a.keys, p.blocks, tokens);
+  auto finalize = [&](auto kernel, unsigned threads) {
+    hipLaunchKernelGGL(kernel, fin, dim3(threads), 0, stream, a.keys, p.blocks, tokens);
+  };
+  if (p.blocks <= 256) finalize(argmax_finalize_kernel<256, 1>, 256);
+  else if (p.blocks <= 1024) finalize(argmax_finalize_kernel<256, 4>, 256);
+  else finalize(argmax_finalize_kernel<1024, 8>, 1024);
   HS_CHECK_LAUNCH("argmax finalize");
   return HS_OK;
 }
