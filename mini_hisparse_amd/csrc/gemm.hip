@@ -339,53 +339,52 @@ static int64_t gemm_ceil(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // Waves of a workgroup: 8 where a wave of 4 would read its k-steps in more than one round
 // (each round is a memory round trip, and a CU with one workgroup has only its own waves'
 // loads in flight), unless there are so many rows that every CU holds several workgroups
-// (then only for steps that fill the 8 waves' first round too).
+// (then only for a long K).
 // 8 rows, us with 4 and with 8 waves: 3584 x 3584 9.8 and 8.5, 896 x 4864 10.5 and 8.3,
-// 3584 x 18944 39.4 and 30.0; 1152 x 896 (7 steps a wave of 4) 3.60 and 3.65; one tile of
-// 12288 x 1536 9.3 and 10.9.  The same for a projection in one K slice and its fused forms,
+// 3584 x 18944 39.4 and 30.0; 1152 x 896 (7 steps a wave of 4) 3.60 and 3.65; 12288 x
+// 1536 9.3 and 10.9, 12288 x 3584, one row, 17.2 and 18.1.  The same for a projection in one K slice and its fused forms,
 // so their sums agree.
 static int gemm_waves(int64_t N, int64_t slice_steps) {
-  return slice_steps > 32 && (N <= 8192 || (slice_steps > 64 && N <= 16384)) ? 8 : 4;
+  return slice_steps > 32 && (N <= 8192 || (slice_steps > 112 && N <= 16384)) ? 8 : 4;
 }
 
 // Row tiles of 16 per workgroup and K slices.  The weight's stream bounds the launch, a CU
 // reads about 23 bytes per ns, and the launch ends with the CU that reads most: the cost of
 // a plan is the rounds of its workgroups over the 256 CUs times a workgroup's tile-steps
-// (1 KB each), an eighth more with one tile, which reads x twice as often per weight byte.
-// A second tile costs about 24 tile-steps (1 us of loads, LDS sums and stores) whatever K is.
-// Merging K slices costs about 48 (2 us), and pays only within one round or for long slices;
-// more than three only while each keeps 96 k-steps (few rows of a long K).
+// (1 KB each) and its x reads: 1/20 tile-step per token row and step, of which a second tile
+// has no more.  A second tile costs about 28 tile-steps (over 1 us of loads, LDS sums and stores)
+// whatever K is.  Merging K slices costs about 48 (2 us), and pays only within one round or for
+// long slices; more than three only while each keeps 80 k-steps (few rows of a long K).  The
+// slices are chosen without the token rows (an eighth of the tile-steps for one tile's x, no
+// charge for the second), so a row's sums are the same in every batch.
 // Measured, 8 rows, us with at least 512 workgroups of 4 waves (one tile up to 16384 rows) and
 // with these plans: 3584 x 18944 34.2 and 28.5 (two tiles in two slices instead of one in
 // three), 7168 x 5120 21.6 and 15.7, 5120 x 27648 64.9 and 53.3 (two tiles in three slices),
 // 896 x 4864 9.6 and 7.5 (three slices); without the second tile's share 8192 x 512 takes two
 // tiles, 4.4 and 5.1, with it one, 4.4; with at most three slices 16 x 27648 12.0 instead of
-// 8.1, with eight 7.5.
-static GemmPlan plan_gemm(int64_t N, int64_t K, bool one_slice = false) {
+// 8.1, with eight 7.5.  The argmax of 152064 x 896, one tile and two: 42.7 and 46.0 for one token
+// row, 51.3 and 47.5 for 8, 66.2 and 52.7 for 16.
+static GemmPlan plan_gemm(int64_t rows, int64_t N, int64_t K, bool one_slice = false) {
   // unsigned, with constant divisors: every projection call plans, on the host's time
-  constexpr uint64_t CUS = 256, X_SHARE = 8, TILE2 = 24, MERGE = 48, LONG_SLICE = 256, MORE_SLICES = 96;
-  const uint64_t steps = static_cast<uint64_t>(K) / 32;
+  constexpr uint64_t CUS = 256, X_SHARE = 8, X_ROWS = 20, TILE2 = 28, MERGE = 48, LONG_SLICE = 256, MORE_SLICES = 80;
+  const uint64_t M = static_cast<uint64_t>(rows), steps = static_cast<uint64_t>(K) / 32;
   const uint64_t n[2] = {(static_cast<uint64_t>(N) + 15) / 16, (static_cast<uint64_t>(N) + 31) / 32};
   const uint64_t slices[GM_SLICES] = {steps, (steps + 1) / 2, (steps + 2) / 3, (steps + 3) / 4, (steps + 4) / 5,
                                       (steps + 5) / 6, (steps + 6) / 7, (steps + 7) / 8};
-  // Many rows of a short K: 20480 x 512 in one tile 7.7 us, in two 6.9
-  const bool two_tiles = N > 16384 && steps <= 16;
-  GemmPlan p{};
-  uint64_t best = UINT64_MAX;
+  // the tile-steps of the busiest CU
+  auto stream_of = [&](uint64_t s, uint64_t tiles) { return (n[tiles - 1] * s + CUS - 1) / CUS * slices[s - 1] * tiles; };
+  auto sliced = [&](uint64_t s, uint64_t tiles) { return s == 1 || n[tiles - 1] * s <= CUS || slices[s - 1] >= LONG_SLICE; };
+  uint64_t splits = 1, best = UINT64_MAX;
   for (uint64_t s = 1; s <= (one_slice ? 1 : GM_SLICES); ++s) {
     const uint64_t slice = slices[s - 1];
     if (slice * (s - 1) >= steps || (s > 3 && slice < MORE_SLICES)) break;  // one would be empty, or too short
-    for (uint64_t tiles = 2; tiles >= (two_tiles ? 2u : 1u); --tiles) {
-      const uint64_t blocks = n[tiles - 1];
-      if (s > 1 && blocks * s > CUS && slice < LONG_SLICE) continue;
-      const uint64_t stream = (blocks * s + CUS - 1) / CUS * slice * tiles;
-      const uint64_t cost = stream + (tiles == 1 ? stream / X_SHARE : TILE2) + (s > 1 ? MERGE : 0);
+    for (uint64_t tiles = s > 3 ? 1 : 2; tiles >= 1; --tiles) {
+      if (!sliced(s, tiles)) continue;
+      const uint64_t stream = stream_of(s, tiles);
+      const uint64_t cost = stream + (tiles == 1 ? stream / X_SHARE : 0) + (s > 1 ? MERGE : 0);
       if (cost >= best) continue;
       best = cost;
-      p.tiles = static_cast<int>(tiles);
-      p.blocks = static_cast<int64_t>(blocks);
-      p.splits = static_cast<int64_t>(s);
-      p.slice_steps = static_cast<int64_t>(slice);
+      splits = s;
     }
   }
   // Where two tiles per workgroup leave CUs idle (4096 < N <= 6144), the rows are dealt evenly
@@ -394,19 +393,35 @@ static GemmPlan plan_gemm(int64_t N, int64_t K, bool one_slice = false) {
   // 12.2 and 10.3 (14.2 and 12.2), 5120 x 5120 15.9 and 13.6 (19.2 and 16.9), 6144 x 4096 13.2
   // and 12.6 (15.9 and 14.5).  Fewer rows than a tile's, or two rounds, do not pay: the second
   // tile's loads cost more than the bytes they leave out (3584 x 3584 in one tile 8.0, in
-  // 14 rows of two 9.7; 9216 x 4096 19.0 and 20.7), so they are charged 36 here, which leaves
-  // K up to 1024 to one tile (5120 x 512 4.2, even rows 4.9; 4608 x 1024 5.2 and 5.5).  Longer
+  // 14 rows of two 9.7; 9216 x 4096 19.0 and 20.7), so they are charged 44 here, which leaves
+  // a short K to one tile (5120 x 512 4.2, even rows 4.9; 4608 x 1024 5.2 and 5.5).  Longer
   // K stays in slices: 5120 x 27648 in three 50.1, in 20 rows 53.3 (but 4608 x 18944, here two
   // whole tiles and one slice, 41.0 and in 18 rows 36.1).
-  constexpr uint64_t EVEN = 36;
-  uint64_t rows = 2 * ((static_cast<uint64_t>(N) + 2 * CUS - 1) / (2 * CUS));
-  if (rows == 22) rows = 24;  // starts at multiples of 2: 22 rows could touch a third tile
-  if (!one_slice && rows > 16 && rows <= 24 && steps <= 2 * LONG_SLICE && steps * rows / 16 + EVEN < best) {
+  constexpr uint64_t EVEN = 44;
+  uint64_t even = 2 * ((static_cast<uint64_t>(N) + 2 * CUS - 1) / (2 * CUS));
+  if (even == 22) even = 24;  // starts at multiples of 2: 22 rows could touch a third tile
+  const bool dealt = !one_slice && even > 16 && even <= 24 && steps <= 2 * LONG_SLICE;
+  if (dealt && steps * even / 16 < best) splits = 1;
+  GemmPlan p{};
+  p.splits = static_cast<int64_t>(splits);
+  p.slice_steps = static_cast<int64_t>(slices[splits - 1]);
+  // Many rows of a short K in two tiles as long as all of these workgroups run at once: 20480 x 128
+  // in one tile 5.9 us, in two 5.0; 27648 x 128 6.2 and 7.4
+  const bool two_tiles = N > 16384 && n[1] <= 3 * CUS && steps <= 16;
+  best = UINT64_MAX;
+  for (uint64_t tiles = 2; tiles >= (two_tiles ? 2u : 1u); --tiles) {
+    if (!sliced(splits, tiles)) continue;
+    const uint64_t stream = stream_of(splits, tiles);
+    const uint64_t cost = stream + stream * M / (X_ROWS * tiles) + (tiles == 2 ? TILE2 : 0);
+    if (cost >= best) continue;
+    best = cost;
+    p.tiles = static_cast<int>(tiles);
+    p.blocks = static_cast<int64_t>(n[tiles - 1]);
+  }
+  if (dealt && splits == 1 && steps * even / 16 + steps * M / X_ROWS + EVEN < best) {
     p.tiles = 2;
-    p.rows = static_cast<int64_t>(rows);
+    p.rows = static_cast<int64_t>(even);
     p.blocks = gemm_ceil(N, p.rows);
-    p.splits = 1;
-    p.slice_steps = static_cast<int64_t>(steps);
   }
   p.waves = gemm_waves(N, p.slice_steps);
   // A weight is read once per step.  Above the 4 MB of an XCD's L2 nothing of it is left
@@ -461,7 +476,7 @@ using namespace hs;
 
 extern "C" int64_t hs_skinny_gemm_workspace_bytes(int64_t rows, int64_t n, int64_t k) {
   if (rows < 1 || n < 1 || k < 32) return 256;
-  const GemmPlan p = plan_gemm(n, k);
+  const GemmPlan p = plan_gemm(rows, n, k);
   // tagged 64-bit partial words and a counter per row tile (the fp32 partials of the
   // two-launch form fit in the same bytes)
   return p.splits > 1 ? p.splits * rows * n * 8 + p.blocks * 8 + 256 : 256;
@@ -477,7 +492,7 @@ static int run_gemm(const void* x, int64_t x_stride, const void* weight, int64_t
   HS_CHECK_ARG(x && weight && out, "null GEMM pointer");
   HS_CHECK_ARG((reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(weight) & 15) == 0,
                "x and weight must be 16-byte aligned");
-  const GemmPlan p = plan_gemm(n, k);
+  const GemmPlan p = plan_gemm(rows, n, k);
   HS_CHECK_ARG(p.blocks <= 0x7fffffff && p.splits <= 65535, "GEMM too large");
   GemmArgs a{};
   a.x = static_cast<const unsigned short*>(x);
@@ -569,7 +584,7 @@ extern "C" int hs_skinny_gemm_swiglu_tiled(const void* x, int64_t x_stride, cons
   a.slice_steps = k / 32;
   a.F = ffn;
   const dim3 grid(static_cast<unsigned>(blocks));
-  const GemmPlan p = plan_gemm(2 * ffn, k, true);  // the plain projection's waves
+  const GemmPlan p = plan_gemm(rows, 2 * ffn, k, true);  // the plain projection's waves
   if (dtype == HS_DTYPE_BF16) launch_swiglu<HS_DTYPE_BF16>(p, grid, a, stream);
   else launch_swiglu<HS_DTYPE_F16>(p, grid, a, stream);
   HS_CHECK_LAUNCH("skinny GEMM swiglu");
@@ -578,7 +593,7 @@ extern "C" int hs_skinny_gemm_swiglu_tiled(const void* x, int64_t x_stride, cons
 
 extern "C" int64_t hs_skinny_gemm_argmax_workspace_bytes(int64_t rows, int64_t n, int64_t k) {
   if (rows < 1 || n < 1 || k < 32) return 256;
-  return plan_gemm(n, k, true).blocks * rows * 8 + 256;
+  return plan_gemm(rows, n, k, true).blocks * rows * 8 + 256;
 }
 
 extern "C" int hs_skinny_gemm_argmax_tiled(const void* x, int64_t x_stride, const void* weight_tiles, int64_t n,
@@ -592,7 +607,7 @@ extern "C" int hs_skinny_gemm_argmax_tiled(const void* x, int64_t x_stride, cons
   HS_CHECK_ARG(x && weight_tiles && tokens, "null GEMM pointer");
   HS_CHECK_ARG((reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(weight_tiles) & 15) == 0,
                "x and weight must be 16-byte aligned");
-  const GemmPlan p = plan_gemm(n, k, true);
+  const GemmPlan p = plan_gemm(rows, n, k, true);
   HS_CHECK_ARG(p.blocks <= 0x7fffffff, "GEMM too large");
   const int64_t need = p.blocks * rows * 8;
   HS_CHECK_ARG(workspace != nullptr && workspace_bytes >= need && (reinterpret_cast<uintptr_t>(workspace) & 7) == 0,

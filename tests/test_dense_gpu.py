@@ -331,10 +331,11 @@ def test_in_kernel_split_merge_replays_from_a_captured_graph(gpu):
 
 # one round of 4 waves and one k-step more (8 waves), the last row counts with 8 waves and the
 # first with 4, one and two row tiles, a weight of 4 MB and a little more, split and whole K:
-# 2, 3, 4, 6 and 8 slices, the last one shorter
+# 3, 4, 7 and 8 slices, the last one shorter
 PLAN_SHAPES = [(512, 1024), (512, 1056), (2048, 1024), (2064, 1024), (4096, 2048), (4112, 2048), (8192, 1056),
-               (8208, 1056), (8208, 2048), (8208, 2080), (16384, 1056), (16384, 2080), (16416, 1056), (16416, 2080),
-               (16384, 512), (16416, 512), (16416, 544), (96, 9600), (16, 8192), (48, 12288), (48, 12256), (16, 18944), (16, 27648)]
+               (8208, 1056), (8208, 3584), (8208, 3616), (16384, 1056), (16384, 3616), (16416, 1056), (16416, 3616),
+               (16384, 512), (16416, 512), (16416, 544), (24608, 512), (96, 9600), (16, 8192), (48, 10240),
+               (48, 10208), (16, 18944), (16, 27648)]
 
 
 @pytest.mark.gpu
@@ -359,12 +360,11 @@ def test_projection_plans_at_their_edges(gpu, rows, n, k):
 
 
 # row counts whose workgroups take 18, 20 or 24 weight rows wherever these start in the 16-row
-# tiles, the counts beside them (a last workgroup of one row, a full one), and K at the
-# shortest and the longest that does so and one step beside them
+# tiles, the counts beside them (a last workgroup of one row, a full one), K too short for it,
+# long enough for 16 token rows and for one, the longest, and one step past that
 WINDOW_SHAPES = [(4096, 64), (4097, 1056), (4608, 64), (4609, 64), (5120, 1024), (5121, 64), (5632, 64), (5640, 1056),
-                 (6144, 64), (6145, 64), (4608, 16384), (4608, 16416), (4096, 1408), (4608, 1024), (4608, 1056),
-                 (4609, 1408), (5120, 1152), (5120, 1184), (5121, 1568), (5632, 1568), (5640, 1568), (6144, 1536),
-                 (6144, 1568), (6145, 1568)]
+                 (6144, 64), (6145, 64), (4608, 16384), (4608, 16416), (4096, 1728), (4608, 1728), (4609, 2016),
+                 (5120, 2016), (5121, 2880), (5632, 2880), (5640, 2880), (6144, 2880), (6145, 2880)]
 
 
 @pytest.mark.gpu
@@ -376,7 +376,7 @@ def test_projection_rows_across_tile_edges(gpu, rows, n, k):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n,k", [(512, 1056), (4096, 1056), (16416, 2080), (48, 12288), (4097, 1408), (6144, 1568)])
+@pytest.mark.parametrize("n,k", [(512, 1056), (4096, 1056), (16416, 2080), (48, 10240), (4097, 1472), (6144, 2400)])
 def test_projection_plans_of_f16(gpu, n, k):
     """One and two tiles, 4 and 8 waves, slices and rows across tile edges in float16."""
     test_linear_matches_an_fp32_reference(gpu, torch.float16, 9, n, k, True)
