@@ -254,7 +254,6 @@ __device__ __forceinline__ int32_t wave_max_i32(int32_t v) {
   return v;
 }
 
-
 // ---- front: bitmaps, hits and protection, miss ranks, victims, LRU reorder
 // (row_index.py:67-113).  LDS: bits[wl] (selected tokens, then hit tokens),
 // needs[wl], prot[wsw].
@@ -1416,10 +1415,12 @@ static int resolve_launch(const hs_resolve_desc* descs, int32_t count, char* wor
     const size_t lds = static_cast<size_t>(front_lds);
     const bool l16 = batch.d[0].lru_i16 != 0;  // the same for every descriptor (validated)
     // The split front where it measured faster: hot regions above 16384 rows or histories
-    // above 40000 tokens (7B layer shape, 32768 rows and 131072 tokens: 21.9 us for its three
+    // above 40000 tokens (7B layer shape, 32768 rows and 131072 tokens: 21.7 us for its three
     // launches against 37.5 us for the one-workgroup front; 32B stress shape, 2048 rows and
-    // 65536 tokens: the resolve stage 4.20 -> 3.47 ms per step; 0.5B layer shape, 13504 rows
-    // and 32768 tokens: 21.7 against 19.3 us, so it keeps the one-workgroup front).
+    // 65536 tokens: the resolve stage 4.20 -> 3.47 ms per step).  At and below the line, us of
+    // the three launches and of the one, without the two more launch gaps: 16 requests of 16384
+    // rows and 32768 tokens 19.5 and 20.5; 0.5B layer shape, 4 of 13504 rows and 32768 tokens 18.9
+    // and 18.2; 4 of 6752 rows 18.6 and 17.6; one of 4096 rows and 8192 tokens 17.8 and 15.9.
     // HS_RESOLVE_SPLIT=0 / 1 forces either way for descriptors that allow it (read per call).
     const char* split_env = getenv("HS_RESOLVE_SPLIT");
     const int split_force = split_env ? atoi(split_env) : -1;

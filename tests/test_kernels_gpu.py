@@ -347,7 +347,7 @@ def test_resolver_row_stats_accumulate(gpu):
         (torch.bfloat16, 40, 16, 2, 3, 20, 6, True, None),  # D not a multiple of 8: strided scorer
         (torch.bfloat16, 64, 16, 16, 1, 256, 8, True, None),  # query tile above the LDS limit
         (torch.bfloat16, 120, 16, 1, 12, 64, 9, True, None),  # two head chunks per KV head
-        (torch.float16, 20000, 16, 1, 2, 32, 64, True, None),  # keys beyond the LDS key buffer
+        (torch.float16, 20000, 16, 1, 2, 32, 64, True, None),  # more pages than a workgroup's registers hold
     ],
 )
 def test_quest_pages_match_oracle(gpu, dtype, pages, P, kv, g, D, top, sink, length):
@@ -414,8 +414,8 @@ def test_quest_scores_bit_exact(gpu, q_dtype, counts, kv, g, D):
                                              (16384, 64, True), (16385, 64, False), (3000, 65, True)])
 def test_quest_topk_with_many_ties_matches_oracle(gpu, pages, top, sink):
     """Bounds and queries of small integers, so that many pages score exactly alike: the
-    radix select's pages equal the oracle's, ties taken from the lowest page (16384 pages
-    keep the keys in LDS; one more reads them from the scores)."""
+    selected pages equal the oracle's, ties taken from the lowest page (16384 pages keep the
+    keys in registers; one more reads them from the scores)."""
     from mini_hisparse_amd.selection import quest_selection
 
     P, kv, g, D = 16, 2, 7, 64
@@ -427,6 +427,7 @@ def test_quest_topk_with_many_ties_matches_oracle(gpu, pages, top, sink):
     expected = oracle.quest_pages(q, lo, hi, length, P, top, keep_sink=sink)
     sel = quest_selection(q.to(gpu), lo.to(gpu), hi.to(gpu), length, P, top, keep_sink=sink)
     np.testing.assert_array_equal(sel.device_pages[:, : expected.shape[1]].cpu().numpy(), expected)
+
 
 def _score_pages(kind, pages, gen):
     """[pages] page values whose scores crowd, spread or repeat (bf16 exact)."""
@@ -539,6 +540,7 @@ def test_union_builder_matches_host_adapter(gpu, pages, P, kv, g, top, length):
         assert counts[k] == len(cols)
         np.testing.assert_array_equal(topk.entries.columns[k, : len(cols)].cpu().numpy(), cols)
         np.testing.assert_array_equal(topk.entries.masks[k, : len(cols)].cpu().numpy().astype(np.int64), masks)
+
 
 @pytest.mark.parametrize(
     "pages,P,kv,g,top,length",
@@ -1069,7 +1071,7 @@ def test_row_read_probe_covers_the_attention_entries(gpu):
     "dtype,P,kv,D,start,tokens",
     [
         (torch.bfloat16, 16, 4, 128, 5, 1),       # a decode token in the middle of a page
-        (torch.bfloat16, 16, 4, 128, 0, 16 * 70 + 3),  # a prefill of 71 pages: two launches of 64 pages
+        (torch.bfloat16, 16, 4, 128, 0, 16 * 70 + 3),  # a prefill of 71 pages: one launch of the long argument block
         (torch.bfloat16, 16, 2, 64, 13, 40),      # starts 3 rows before a page boundary
         (torch.float16, 7, 2, 24, 3, 30),         # 96-byte rows
         (torch.float32, 4, 1, 8, 2, 11),          # the reference tests' shape
