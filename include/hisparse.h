@@ -122,8 +122,8 @@ int hs_uniform_pages(uint64_t seed, uint64_t step, const int64_t* page_counts, i
  * Replaces: Selection.from_pages (selection.py:43-60) followed by
  * LogicalTopK.from_selection (row_index.py:20-31), without the host sync of
  * selection.py:100.
- *   pages         [batch, heads, top] from hs_quest_topk; lengths host [batch], each at
- *                 most 2^31 - 1 (positions are 32-bit)
+ *   pages         [batch, heads, top] from hs_quest_topk, at most 2^22 heads; lengths host
+ *                 [batch], each at most 2^31 - 1 (positions are 32-bit)
  *   positions     [batch, pos_capacity] int32: ascending union of the
  *                 selected tokens, then -1
  *   head_columns  [batch, heads, width] int64: union column of each head's
@@ -508,8 +508,8 @@ int hs_skinny_gemm_swiglu_tiled(const void* x, int64_t x_stride, const void* gat
  * (-0 equal to +0; a NaN above every number), as torch.argmax over the logits of
  * hs_skinny_gemm_tiled with one K slice -- without writing the logits.  W packed as
  * for hs_skinny_gemm_tiled, n < 2^31.  Each workgroup leaves its best key per token
- * in the workspace (hs_skinny_gemm_argmax_workspace_bytes, 8-byte aligned) and a
- * second launch reduces them.  Replaces the logits GEMM and `argmax` of the
+ * in the workspace (hs_skinny_gemm_argmax_workspace_bytes, 8-byte aligned; one of more
+ * rows serves fewer) and a second launch reduces them.  Replaces the logits GEMM and `argmax` of the
  * reference's greedy decode (engine.py:71-72, _emit: logits.argmax()).
  */
 int64_t hs_skinny_gemm_argmax_workspace_bytes(int64_t rows, int64_t n, int64_t k);

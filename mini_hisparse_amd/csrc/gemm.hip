@@ -593,7 +593,9 @@ extern "C" int hs_skinny_gemm_swiglu_tiled(const void* x, int64_t x_stride, cons
 
 extern "C" int64_t hs_skinny_gemm_argmax_workspace_bytes(int64_t rows, int64_t n, int64_t k) {
   if (rows < 1 || n < 1 || k < 32) return 256;
-  return plan_gemm(rows, n, k, true).blocks * rows * 8 + 256;
+  // one tile per workgroup, the most keys of any row count: a workspace serves fewer rows too, whose
+  // plan may have the smaller workgroups
+  return gemm_ceil(n, 16) * rows * 8 + 256;
 }
 
 extern "C" int hs_skinny_gemm_argmax_tiled(const void* x, int64_t x_stride, const void* weight_tiles, int64_t n,

@@ -383,6 +383,25 @@ def test_projection_plans_of_f16(gpu, n, k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,k", [(300, 8192), (3584, 18944), (16400, 1056), (42391, 896), (16384, 3616)])
+def test_a_workspace_of_more_rows_serves_fewer(gpu, n, k):
+    """The plans of fewer token rows may take other workgroups: what 16 rows need holds them."""
+    from mini_hisparse_amd.dense import (
+        argmax_workspace_bytes, gemm_workspace_bytes, linear_argmax_tiled, linear_tiled, tile_weight,
+    )
+
+    gen = torch.Generator(device=gpu).manual_seed(n + k)
+    x = torch.randn(16, k, generator=gen, device=gpu).to(torch.bfloat16)
+    tiles = tile_weight((torch.randn(n, k, generator=gen, device=gpu) / k**0.5).to(torch.bfloat16))
+    ws = torch.empty(gemm_workspace_bytes(16, n, k), dtype=torch.uint8, device=gpu)
+    argmax_ws = torch.empty(argmax_workspace_bytes(16, n, k), dtype=torch.uint8, device=gpu)
+    y, tokens = linear_tiled(x, tiles, n, workspace=ws), linear_argmax_tiled(x, tiles, n, workspace=argmax_ws)
+    for rows in range(1, 16):  # and a row has the same bits in every batch
+        assert torch.equal(linear_tiled(x[:rows], tiles, n, workspace=ws), y[:rows])
+        assert torch.equal(linear_argmax_tiled(x[:rows], tiles, n, workspace=argmax_ws), tokens[:rows])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n", [16, 4096, 4112, 16384, 24608, 131072, 131088])
 def test_argmax_key_counts(gpu, n):
     """The argmax's last step at one key per token, the most and one more that take one load of
