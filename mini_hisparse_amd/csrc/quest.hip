@@ -954,13 +954,12 @@ __global__ __launch_bounds__(UT) __attribute__((amdgpu_num_sgpr(80))) void build
   const bool masks_in_lds = g * k <= UMAXMASK;
   // a list has at most the history's tokens and at most those of the pages its heads select
   const int64_t c0 = static_cast<int64_t>(chunk) * a.chunk;
-  const int64_t most = static_cast<int64_t>(position ? Hq : g) * k * P;
-  if (position && c0 > 0 && (c0 >= L || c0 >= most)) {
+  if (chunk > 0 && (position || group) && (c0 >= L || c0 >= static_cast<int64_t>(position ? Hq : g) * k * P)) {
+    if (group) return;
     const int64_t end = c0 + a.chunk < a.pos_cap ? c0 + a.chunk : a.pos_cap;
     for (int64_t i = c0 + T; i < end; i += UT) a.positions[b * a.pos_cap + i] = -1;
     return;
   }
-  if (group && c0 > 0 && (c0 >= L || c0 >= most)) return;
   // page and row of a token offset: a shift where the page size is a power of two
   auto page_of = [&](uint32_t i) { return static_cast<int32_t>(a.pshift >= 0 ? i >> a.pshift : i / static_cast<uint32_t>(P)); };
 
@@ -971,9 +970,12 @@ __global__ __launch_bounds__(UT) __attribute__((amdgpu_num_sgpr(80))) void build
   if (group && masks_in_lds)
     for (int32_t i = T; i < g * k; i += UT) gmask[i] = 0u;
   __syncthreads();
-  // the thread's pages, UT apart; heads times pages may pass 31 bits, so head and page are stepped
-  const int32_t step_h = UT / k, step_j = UT - step_h * k;
-  for (int32_t h = T / k, j = T - h * k; h < Hq;) {
+  // the thread's pages, UT apart; heads times pages may pass 31 bits, so head and page are stepped.
+  // The quotients of up to UT by k come from a reciprocal of one ulp: half a step off the integers
+  // is 2^-11 of them or more (an integer division of each took 0.2 us a launch).
+  const float by_k = __builtin_amdgcn_rcpf(static_cast<float>(k));
+  const int32_t step_h = static_cast<int32_t>((UT + 0.5f) * by_k), step_j = UT - step_h * k;
+  for (int32_t h = static_cast<int32_t>((T + 0.5f) * by_k), j = T - h * k; h < Hq;) {
     const int32_t p = pg[h * top + j];
     if (p >= 0 && p < count) {
       atomicOr(&ubits[p >> 5], 1u << (p & 31));
